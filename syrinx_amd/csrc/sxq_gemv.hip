@@ -1250,6 +1250,7 @@ hipError_t launch_gemv(const QWeight& w, const void* act, int m, float* y, int64
         if (fits && m <= 4) return gemv2_dispatch<4>(w, act, m, y, ldy, bias, res, ldr, s);
         // 5..16 rows of Q4_K: one pass over the weights on the matrix cores
         if (w.dtype == kQ4K && m <= 16 && gemv_mma_on()) return gemv_mma_launch(w, act, m, y, ldy, bias, res, ldr, s);
+        if (w.dtype != kQ4K && m >= kGemmQ80MinRows) return launch_gemm_q80(w, act, m, y, ldy, bias, res, ldr, s);
         // 5..16 rows: the task-split kernel four activation rows at a time (each launch
         // streams the weights again; per row this is still well ahead of the
         // one-group-per-row kernel, whose few waves leave most of the GPU idle).

@@ -417,7 +417,7 @@ sxq_status check_config(const sxq_lm_config* c) {
 
 // One projection of T prompt rows: x_f32 [T][k] (f32 rows) and act (the same rows as
 // device activation blocks) -> y [T][n] (+ bias, then res + that).  Q4_K: the f16 MFMA GEMM
-// from kGemmMinRows rows unless `exact`; Q8_0 / Q4_0: the int8 matrix-core GEMM from
+// from kGemmMinRows rows unless `exact`; Q8_0 / Q4_0: the int8 matrix cores from
 // kGemmQ80MinRows rows; otherwise the GEMV, 16 rows at a time (Candle's bits).
 hipError_t pf_proj(const sxq_lm* lm, const QWeight& w, const float* x, const uint8_t* act, int T, float* y,
                    const float* bias, const float* res, bool exact, void* gemm_ws, hipStream_t s) {

@@ -46,3 +46,27 @@ def test_quantize_rows_remainders_and_unaligned(cuda, ora, dt, k, n, shift):
     want = ora.quantize(int(dt), x).reshape(-1)
     np.testing.assert_array_equal(got[shift: shift + nbytes], want)
     assert (got[:shift] == 0xA5).all() and (got[shift + nbytes:] == 0xA5).all()
+
+
+# (n, k, m): weight tiles of 16 / 64 / 128 rows and row tiles of 16 / 32 / 64 with remainders,
+# block counts below, at and past a chunk (4, 8, 16, 32 blocks), each kernel of the dispatch
+Q80_SHAPES = [(1, 32, 5), (17, 320, 16), (16, 1024, 17), (130, 1056, 33), (896, 4864, 8), (77, 992, 64), (200, 160, 65),
+              (1152, 896, 226), (2048, 1024, 500), (4100, 96, 130), (896, 4864, 226), (9728, 896, 50), (64, 2080, 300)]
+
+
+@pytest.mark.parametrize("dt", [G.Q8_0, G.Q4_0])
+@pytest.mark.parametrize("n,k,m", Q80_SHAPES)
+def test_q80_matrix_core_bit_exact(cuda, ora, dt, n, k, m):
+    """Five rows and more of Q8_0 / Q4_0: Candle's bits, with a bias and zero / tied rows."""
+    rng = np.random.default_rng(n + k + m)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    w[0] = 0.0
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[1] = 0.0
+    x[2, :32] = -3.0
+    b = rng.standard_normal(n).astype(np.float32)
+    blocks = ora.quantize(int(dt), w)
+    qmm = QMatMul.from_qtensor(QTensor.from_blocks(blocks, (n, k), dt, device=cuda))
+    got = qmm.forward(torch.from_numpy(x).to(cuda), bias=torch.from_numpy(b).to(cuda)).cpu().numpy()
+    want = (ora.matmul(int(dt), x, blocks) + b[None, :]).astype(np.float32)
+    assert (got == want).all(), f"{int((got != want).sum())} of {got.size} outputs differ"
