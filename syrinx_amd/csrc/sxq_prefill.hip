@@ -43,113 +43,144 @@ __global__ __launch_bounds__(64) void k_prefill_rope_kv(const float* __restrict_
 }
 
 constexpr int kPfRows = 64;  // query rows (tokens x heads of one KV group) per workgroup
-constexpr int kPfKeys = 32;  // key positions per LDS block
+constexpr int kPfKeys = 64;  // key positions per LDS tile: 32 for each half of the waves
 
+// LDS row strides (floats): a lane's float4 reads of 16 consecutive keys, and the value reads
+// of 32 dims of two keys four apart, each hit every bank once.
+constexpr int pf_kstride(int hd) { return hd + 4; }
+constexpr int pf_vstride(int hd) { return hd + 8; }
 size_t prefill_attn_lds(int hd) {
-    return sizeof(float) * ((size_t)(kPfRows + 2 * kPfKeys) * (hd + 4) + (size_t)kPfRows * (kPfKeys + 1));
+    const size_t tiles = sizeof(float) * (size_t)kPfKeys * (pf_kstride(hd) + pf_vstride(hd));
+    const size_t merge = sizeof(float) * 2 * 64 * (size_t)(hd / 2 + 2);  // two waves' accumulators, m and l
+    return tiles > merge ? tiles : merge;
 }
+
+typedef float v16f __attribute__((ext_vector_type(16)));
 
 // One workgroup (256 threads) per (tile, KV group): a tile is up to kPfRows / G
 // consecutive prompt tokens of one stream (tile = {stream, first token row t0, count,
 // position p0 of token t0}); its rows are r = i * G + hh (token i, query head g * G + hh).
-// Keys stream through LDS in blocks of kPfKeys positions (0 .. p0 + count - 1); every row
-// keeps an online softmax (running max m, sum l, rescaled accumulator), masking keys past
-// its own position.  Thread (r, qd) = (tid / 4, tid % 4) scores keys 8 qd .. 8 qd + 7 of a
-// block for row r and accumulates head dims qd * HD/4 .. +HD/4 - 1 of that row.
+// Everything is f32 on the f32 matrix cores (v_mfma_f32_32x32x2_f32), transposed so that a
+// row's softmax stays in its lane: wave w holds rows 32 (w & 1) .. +31 and takes the 32-key
+// halves w >> 1 of the tiles; lane (c, h) = (lane & 31, lane >> 5) owns row c.
+//   scores^T = K Q^T: result i of a lane is key 8 (i / 4) + 4 h + i % 4 of its row (the query
+//     row is in the lane's registers for the whole kernel; K's dims are taken in the order 8 u
+//     + 4 h + t, so that a lane reads float4s);
+//   out^T += V^T P^T: the probabilities are already the operand the product needs (MFMA i takes
+//     that key from half h), V comes from LDS a row of 32 dims at a time.
+// Each wave keeps an online softmax (running max m, sum l, rescaled accumulator) over its own
+// keys, masking keys past a row's own position; the two halves' results meet in LDS at the end.
+// Bound by the f32 matrix cores (64 cycles per 4096 flops): 1412 ragged tokens of 32 / 8 heads of
+// 128 in 196 us per layer, 226 tokens of 14 / 2 heads of 64 in 21.4 us; with the same tiles
+// on the VALU (a score per thread, four threads per row) 591 and 66 us.  Tiles are taken last
+// first: the last tokens of a prompt attend the most keys.
 template <int HD>
-__global__ __launch_bounds__(256) void k_prefill_attn(const float* __restrict__ q, const float* __restrict__ kc,
-                                                      const float* __restrict__ vc, const int4* __restrict__ tiles,
-                                                      int nh, int nkv, int max_seq, int64_t kv_stream_stride,
-                                                      float scale, float* __restrict__ ctx) {
+__global__ __launch_bounds__(256, 2) void k_prefill_attn(const float* __restrict__ q, const float* __restrict__ kc,
+                                                         const float* __restrict__ vc, const int4* __restrict__ tiles,
+                                                         int nh, int nkv, int max_seq, int64_t kv_stream_stride,
+                                                         float scale, float* __restrict__ ctx) {
     extern __shared__ float4 smem4[];
-    constexpr int hdp = HD + 4, DPT = HD / 4;
-    const int4 tl = tiles[blockIdx.x];
+    constexpr int KS = pf_kstride(HD), VS = pf_vstride(HD), U = HD / 8, DG = HD / 32;
+    const int4 tl = tiles[gridDim.x - 1 - blockIdx.x];
     const int s = tl.x, t0 = tl.y, cnt = tl.z, p0 = tl.w;
     const int g = blockIdx.y, G = nh / nkv, R = cnt * G;
-    float* qs = (float*)smem4;          // [kPfRows][hdp]
-    float* kt = qs + kPfRows * hdp;     // [kPfKeys][hdp]
-    float* vt = kt + kPfKeys * hdp;     // [kPfKeys][hdp]
-    float* pr = vt + kPfKeys * hdp;     // [kPfRows][kPfKeys + 1] probabilities of the block
-    const int tid = threadIdx.x, r = tid >> 2, qd = tid & 3;
-    const int qrow = nh * HD;  // floats per token row of q and ctx
-    for (int e = tid; e < kPfRows * HD; e += 256) {
-        const int rr = e / HD, d = e - rr * HD;
-        float v = 0.0f;
-        if (rr < R) v = q[(int64_t)(t0 + rr / G) * qrow + (g * G + rr % G) * HD + d];
-        qs[rr * hdp + d] = v;
-    }
-    const bool live = r < R;
-    const int qpos = live ? p0 + r / G : -1;
-    float m = -INFINITY, l = 0.0f, acc[DPT];
+    float* kt = (float*)smem4;      // [kPfKeys][KS]
+    float* vt = kt + kPfKeys * KS;  // [kPfKeys][VS]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = lane & 31, h = lane >> 5, half = wave >> 1;
+    const int row = 32 * (wave & 1) + c;
+    const int rr = min(row, R - 1);  // rows past the tile compute on a copy and store nothing
+    const int64_t qoff = (int64_t)(t0 + rr / G) * nh * HD + (g * G + rr % G) * HD;
+    const int qpos = p0 + rr / G;
+    float4 qv[U];
 #pragma unroll
-    for (int i = 0; i < DPT; ++i) acc[i] = 0.0f;
+    for (int u = 0; u < U; ++u) qv[u] = *(const float4*)(q + qoff + 8 * u + 4 * h);
+    float m = -INFINITY, l = 0.0f;
+    v16f o[DG];
+#pragma unroll
+    for (int d = 0; d < DG; ++d) o[d] = v16f{};
     const int64_t koff = (int64_t)s * kv_stream_stride + (int64_t)g * max_seq * HD;
     const int kend = p0 + cnt;
     for (int j0 = 0; j0 < kend; j0 += kPfKeys) {
-        const int nk = min(kPfKeys, kend - j0);
-        __syncthreads();  // the previous block's K, V and P are no longer read
-        load_kv_tile(kt, vt, kc + koff + (int64_t)j0 * HD, vc + koff + (int64_t)j0 * HD, nk, HD);
-        __syncthreads();
-        float sc[8];
-#pragma unroll
-        for (int jj = 0; jj < 8; ++jj) sc[jj] = 0.0f;
-        const float* qr = qs + r * hdp;
-        for (int d = 0; d < HD; d += 4) {
-            const float4 qv = *(const float4*)(qr + d);
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                const float4 kv = *(const float4*)(kt + (8 * qd + jj) * hdp + d);
-                sc[jj] += qv.x * kv.x;
-                sc[jj] += qv.y * kv.y;
-                sc[jj] += qv.z * kv.z;
-                sc[jj] += qv.w * kv.w;
+        lds_barrier();  // the previous tile is no longer read
+        for (int e = tid; e < kPfKeys * (HD / 4); e += 256) {
+            const int key = e / (HD / 4), d = 4 * (e % (HD / 4));
+            float4 kv = make_float4(0.f, 0.f, 0.f, 0.f), vv = kv;
+            if (j0 + key < kend) {
+                kv = *(const float4*)(kc + koff + (int64_t)(j0 + key) * HD + d);
+                vv = *(const float4*)(vc + koff + (int64_t)(j0 + key) * HD + d);
             }
+            *(float4*)(kt + key * KS + d) = kv;
+            *(float4*)(vt + key * VS + d) = vv;
+        }
+        lds_barrier();
+        const int jb = j0 + 32 * half;  // this wave's first key
+        if (jb >= kend) continue;       // uniform per wave; every wave reaches each barrier
+        v16f sc = v16f{};
+        const float* kr = kt + (32 * half + c) * KS + 4 * h;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float4 kv = *(const float4*)(kr + 8 * u);
+            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qv[u].x, sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qv[u].y, sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qv[u].z, sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qv[u].w, sc, 0, 0, 0);
         }
         float bm = -INFINITY;
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-            const int j = 8 * qd + jj;
-            const bool ok = live && j < nk && j0 + j <= qpos;
-            sc[jj] = ok ? sc[jj] * scale + 0.0f : -INFINITY;
-            bm = fmaxf(bm, sc[jj]);
+        for (int i = 0; i < 16; ++i) {
+            const int j = jb + 8 * (i >> 2) + 4 * h + (i & 3);
+            sc[i] = j <= qpos ? sc[i] * scale + 0.0f : -INFINITY;
+            bm = fmaxf(bm, sc[i]);
         }
-        bm = fmaxf(bm, __shfl_xor(bm, 1, 64));
-        bm = fmaxf(bm, __shfl_xor(bm, 2, 64));
+        bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
         const float mn = fmaxf(m, bm);
         const float corr = mn == -INFINITY ? 1.0f : expf(m - mn);
         float ps = 0.0f;
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-            const float p = sc[jj] == -INFINITY ? 0.0f : expf(sc[jj] - mn);
-            pr[r * (kPfKeys + 1) + 8 * qd + jj] = p;
-            ps += p;
+        for (int i = 0; i < 16; ++i) {
+            sc[i] = sc[i] == -INFINITY ? 0.0f : expf(sc[i] - mn);
+            ps += sc[i];
         }
-        ps += __shfl_xor(ps, 1, 64);
-        ps += __shfl_xor(ps, 2, 64);
+        ps += __shfl_xor(ps, 32, 64);
         l = l * corr + ps;
         m = mn;
-        __syncthreads();  // the row's probabilities (written by its four threads) are visible
+        const float* vr = vt + (32 * half + 4 * h) * VS + c;
 #pragma unroll
-        for (int i = 0; i < DPT; ++i) acc[i] *= corr;
-        const float* prow = pr + r * (kPfKeys + 1);
-        for (int j = 0; j < nk; ++j) {
-            const float p = prow[j];
-            const float* vr = vt + j * hdp + qd * DPT;
+        for (int d = 0; d < DG; ++d) {
 #pragma unroll
-            for (int i = 0; i < DPT; i += 4) {
-                const float4 v = *(const float4*)(vr + i);
-                acc[i] += p * v.x;
-                acc[i + 1] += p * v.y;
-                acc[i + 2] += p * v.z;
-                acc[i + 3] += p * v.w;
-            }
+            for (int i = 0; i < 16; ++i) o[d][i] *= corr;
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[(8 * (i >> 2) + (i & 3)) * VS + 32 * d], sc[i], o[d], 0, 0, 0);
         }
     }
-    if (!live) return;
-    float* out = ctx + (int64_t)(t0 + r / G) * qrow + (g * G + r % G) * HD + qd * DPT;
+    // the second half's waves hand their rows to the first half's
+    lds_barrier();
+    float* ex = (float*)smem4 + (wave & 1) * 64 * (HD / 2 + 2);
+    if (half == 1) {
 #pragma unroll
-    for (int i = 0; i < DPT; i += 4)
-        *(float4*)(out + i) = make_float4(acc[i] / l, acc[i + 1] / l, acc[i + 2] / l, acc[i + 3] / l);
+        for (int d = 0; d < DG; ++d)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) ex[(16 * d + i) * 64 + lane] = o[d][i];
+        ex[(HD / 2) * 64 + lane] = m;
+        ex[(HD / 2 + 1) * 64 + lane] = l;
+    }
+    lds_barrier();
+    if (half == 1 || row >= R) return;
+    const float m1 = ex[(HD / 2) * 64 + lane], l1 = ex[(HD / 2 + 1) * 64 + lane];
+    const float mn = fmaxf(m, m1);
+    const float c0 = mn == -INFINITY ? 1.0f : expf(m - mn), c1 = mn == -INFINITY ? 1.0f : expf(m1 - mn);
+    const float lt = l * c0 + l1 * c1;
+#pragma unroll
+    for (int d = 0; d < DG; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) {
+            float v[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) v[t] = (o[d][i + t] * c0 + ex[(16 * d + i + t) * 64 + lane] * c1) / lt;
+            *(float4*)(ctx + qoff + 32 * d + 2 * i + 4 * h) = make_float4(v[0], v[1], v[2], v[3]);
+        }
 }
 
 // One thread per token t (and per tile index): stream-major order, stream s's tokens at

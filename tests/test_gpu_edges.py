@@ -12,6 +12,7 @@ from syrinx_amd._lib import check, lib
 pytestmark = pytest.mark.gpu
 
 G = GgmlDType
+G_Q8 = GgmlDType.Q8_0
 
 
 @pytest.fixture(scope="module")
@@ -70,3 +71,63 @@ def test_q80_matrix_core_bit_exact(cuda, ora, dt, n, k, m):
     got = qmm.forward(torch.from_numpy(x).to(cuda), bias=torch.from_numpy(b).to(cuda)).cpu().numpy()
     want = (ora.matmul(int(dt), x, blocks) + b[None, :]).astype(np.float32)
     assert (got == want).all(), f"{int((got != want).sum())} of {got.size} outputs differ"
+
+
+@pytest.mark.parametrize("n,k,m", [(7, 256, 17), (40, 1536, 33), (1003, 2560, 63), (6144, 512, 48), (130, 1024, 21)])
+def test_q4k_slabs_bit_exact(cuda, ora, n, k, m):
+    """17..63 rows of Q4_K (and any count with exact=True): every 16-row slab of one launch, a
+    partial last slab, weight tiles that are no multiple of eight."""
+    rng = np.random.default_rng(n + k + m)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    x = rng.standard_normal((m + 100, k)).astype(np.float32)
+    b = rng.standard_normal(n).astype(np.float32)
+    blocks = ora.quantize(ora.Q4K, w)
+    qmm = QMatMul.from_qtensor(QTensor.from_blocks(blocks, (n, k), G.Q4K, device=cuda))
+    want = (ora.matmul(ora.Q4K, x, blocks) + b[None, :]).astype(np.float32)
+    bias = torch.from_numpy(b).to(cuda)
+    assert (qmm.forward(torch.from_numpy(x[:m]).to(cuda), bias=bias).cpu().numpy() == want[:m]).all()
+    assert (qmm.forward(torch.from_numpy(x).to(cuda), bias=bias, exact=True).cpu().numpy() == want).all()
+
+
+@pytest.mark.parametrize("dt,k", [(G.Q4K, 512), (G.Q8_0, 96), (G.Q4_0, 320)])
+@pytest.mark.parametrize("m", [2, 7, 40])
+def test_bf16_rows_quantized_directly(cuda, dt, k, m):
+    """bf16 x through the quantizer equals the f32 x of the same values, bit for bit, also from
+    a base that is not 8-byte aligned."""
+    g = torch.Generator(device=cuda).manual_seed(k + m)
+    qmm = QMatMul.from_qtensor(QTensor.quantize(torch.randn(100, k, generator=g, device=cuda) * 0.02, dt))
+    buf = torch.randn(m * k + 1, generator=g, device=cuda).bfloat16()
+    for x in (buf[:-1].view(m, k), buf[1:].view(m, k)):
+        assert torch.equal(qmm.forward(x), qmm.forward(x.float()))
+
+
+@pytest.mark.parametrize("hd,G,nkv", [(128, 4, 2), (64, 7, 2), (128, 1, 2), (64, 64, 1), (128, 5, 1)])
+def test_prefill_attention_tiles(cuda, hd, G, nkv):
+    """Causal attention of ragged prompts on top of filled caches against 64 bits: prompts of one
+    token, of a partial and of several row tiles, caches that end inside a key tile."""
+    from syrinx_amd.decoder import DecoderConfig, DecoderLM
+    cfg = DecoderConfig(n_layers=1, dim=256, n_heads=G * nkv, n_kv_heads=nkv, head_dim=hd, intermediate=256, vocab=64,
+                        max_seq=330, max_batch=4, weight_dtype=int(G_Q8), tied_embedding=0, qk_norm=0)
+    lm = DecoderLM(cfg, device=cuda)
+    lm.init_random(seed=5, std=0.05)
+    gen = torch.Generator(device=cuda).manual_seed(hd + G)
+    for counts in ([1, 31, 64, 130], [70, 33, 1, 65]):  # the second call starts at the first's lengths
+        pos0 = lm.lengths(4)
+        xs = [torch.randn(c, cfg.dim, generator=gen, device=cuda) * 3 for c in counts]
+        tr = lm.prefill(embeds=xs, all_logits=True, trace=True)[3]["layers"][0]
+        q = torch.from_numpy(tr["q"]).to(cuda).double().view(-1, G * nkv, hd)
+        got = torch.from_numpy(tr["ctx"]).to(cuda).double().view(-1, G * nkv, hd)
+        at = 0
+        for s, c in enumerate(counts):
+            for g in range(nkv):
+                k, v = (t.double() for t in lm.read_kv(0, s, g, 0, pos0[s] + c))
+                mask = torch.arange(pos0[s] + c, device=cuda)[None, :] > pos0[s] + torch.arange(c, device=cuda)[:, None]
+                for h in range(G):
+                    sc = (q[at:at + c, g * G + h] @ k.t() / hd ** 0.5).masked_fill(mask, float("-inf"))
+                    want = torch.softmax(sc, -1) @ v
+                    # f32 scores of magnitude |s| err by ~|s| 2^-24 sqrt(hd), which the exponential
+                    # passes on to the weights; the weighted sum errs by about as much again
+                    tol = 8 * 2.0 ** -24 * (sc[~mask].abs().max() + 4) * hd ** 0.5 * v.abs().max()
+                    err = (got[at:at + c, g * G + h] - want).abs().max()
+                    assert err <= tol, f"counts {counts} stream {s} head {g * G + h}: {float(err):.3g} > {float(tol):.3g}"
+            at += c
