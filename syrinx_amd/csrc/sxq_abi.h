@@ -44,7 +44,8 @@ struct FwdPlan {
     int vdt = 0;
     int64_t nbv = 0;    // activation blocks per row
     size_t ws = 0;      // device workspace: activation blocks, or the GEMM's staging
-    size_t xconv = 0;   // SXQ_BF16_INPUT: the f32 copy of x at the workspace's end (inside ws)
+    bool bf16 = false;  // SXQ_BF16_INPUT
+    size_t xconv = 0;   // the f32 copy of a bf16 x at the workspace's end (inside ws), where the kernels need one
 };
 // Candle's argument checks of QMatMul::forward (its error texts), then the plan; flags
 // outside `allowed` are rejected.

@@ -291,6 +291,12 @@ sxq_status sxq_qmm_destroy(sxq_qmm* q) {
 namespace sxq {
 namespace abi {
 
+// Whether a one-row forward runs the GEMV that quantizes x in its prologue.
+static bool fused_quant(const QWeight& w) {
+    static const bool separate = getenv("SXQ_GEMV_QUANT_SEPARATE") != nullptr;  // A/B: two launches
+    return w.dtype != kQ4K && !separate && gemv_quant_fits(w);
+}
+
 sxq_status plan_forward(const sxq_qmm* q, const int64_t* shape, int ndim, const int64_t* strides, unsigned flags,
                         unsigned allowed, FwdPlan* p) {
     if (!q) return fail(SXQ_ERR_INVALID, "qmm_forward: null handle");
@@ -328,8 +334,12 @@ sxq_status plan_forward(const sxq_qmm* q, const int64_t* shape, int ndim, const 
     p->ws = m == 0 ? 0
                    : up256(p->gemm && !q80 ? gemm_q4k_workspace(q->w.n, (int)m, q->w.k)
                                            : (size_t)m * (size_t)p->nbv * act_block_bytes(p->vdt));
-    // bf16 input: widened to f32 at the workspace's end, then the f32 forward
-    p->xconv = (flags & SXQ_BF16_INPUT) && m > 0 ? up256((size_t)m * (size_t)q->w.k * 4) : 0;
+    // bf16 input: the quantizer reads it (an exact widening in registers: no launch and no f32
+    // copy of x).  The f16 GEMM and the one-row GEMV that quantizes in its prologue take f32
+    // rows: widened to f32 at the workspace's end, then the f32 forward.
+    p->bf16 = (flags & SXQ_BF16_INPUT) && m > 0;
+    const bool f32_rows = (p->gemm && !q80) || (m == 1 && fused_quant(q->w));
+    p->xconv = p->bf16 && f32_rows ? up256((size_t)m * (size_t)q->w.k * 4) : 0;
     p->ws += p->xconv;
     return SXQ_OK;
 }
@@ -349,15 +359,12 @@ hipError_t run_forward(const sxq_qmm* q, const FwdPlan& p, const float* x, float
         return e;
     }
     // one row of Q8_0 / Q4_0: the GEMV quantizes x in its own prologue (one launch, same bits)
-    static const bool separate = getenv("SXQ_GEMV_QUANT_SEPARATE") != nullptr;  // A/B: two launches
-    if (m == 1 && !p.gemm && !separate && gemv_quant_fits(q->w)) return launch_gemv_quant(q->w, x, y, bias, nullptr, s);
-    hipError_t e = launch_quantize_act(p.vdt, false, x, k, (int)m, (int)k, ws, s);
-    if (p.gemm) return e == hipSuccess ? launch_gemm_q80(q->w, ws, (int)m, y, n, bias, nullptr, 0, s) : e;
-    for (int64_t r0 = 0; r0 < m && e == hipSuccess; r0 += 16) {
-        const int mm = (int)(m - r0 < 16 ? m - r0 : 16);
-        e = launch_gemv(q->w, ws + (size_t)r0 * p.nbv * act_block_bytes(p.vdt), mm, y + r0 * n, n, bias, nullptr, 0, s);
-    }
-    return e;
+    if (m == 1 && fused_quant(q->w)) return launch_gemv_quant(q->w, x, y, bias, nullptr, s);
+    hipError_t e = p.bf16 ? launch_quantize_act_bf16(p.vdt, (const uint16_t*)(const void*)x, k, (int)m, (int)k, ws, s)
+                          : launch_quantize_act(p.vdt, false, x, k, (int)m, (int)k, ws, s);
+    if (e != hipSuccess) return e;
+    return p.gemm ? launch_gemm_q80(q->w, ws, (int)m, y, n, bias, nullptr, 0, s)
+                  : launch_gemv(q->w, ws, (int)m, y, n, bias, nullptr, 0, s);
 }
 
 }  // namespace abi

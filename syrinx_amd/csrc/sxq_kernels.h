@@ -8,6 +8,9 @@ namespace sxq {
 // canon = Candle's block bytes; otherwise the device layout (ActQ8K / ActQ8_0).
 hipError_t launch_quantize_act(int vdt, bool canon, const float* x, int64_t ldx, int m, int k, void* out,
                                hipStream_t s);
+// The device layout from bf16 rows (each value widened exactly): the blocks of the f32 rows
+// holding the same values.
+hipError_t launch_quantize_act_bf16(int vdt, const uint16_t* x, int64_t ldx, int m, int k, void* out, hipStream_t s);
 // Weight quantization (QTensor::quantize): x [nblocks * bs] -> canonical blocks.
 hipError_t launch_from_float(int dt, const float* x, int64_t nblocks, void* out, hipStream_t s);
 // Dequantization (QTensor::dequantize) of canonical blocks.
@@ -25,7 +28,7 @@ struct QWeight {
     const uint8_t* qs = nullptr;   // Q4_K: 128 B; Q8_0: 32 B; Q4_0: 16 B per block
 };
 
-// Decode GEMV, m in 1..16: y[m, n] (row stride ldy) = act[m] . W^T (+ bias) and, if
+// Decode GEMV, any m: y[m, n] (row stride ldy) = act[m] . W^T (+ bias) and, if
 // `res` is given, y = res + that (res may alias y: each element is read then written
 // by one lane).  act is the device activation layout [m][nb] (ActQ8K for Q4_K,
 // ActQ8_0 otherwise).

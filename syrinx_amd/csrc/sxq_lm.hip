@@ -418,7 +418,7 @@ sxq_status check_config(const sxq_lm_config* c) {
 // One projection of T prompt rows: x_f32 [T][k] (f32 rows) and act (the same rows as
 // device activation blocks) -> y [T][n] (+ bias, then res + that).  Q4_K: the f16 MFMA GEMM
 // from kGemmMinRows rows unless `exact`; Q8_0 / Q4_0: the int8 matrix cores from
-// kGemmQ80MinRows rows; otherwise the GEMV, 16 rows at a time (Candle's bits).
+// kGemmQ80MinRows rows; otherwise the GEMV (Candle's bits).
 hipError_t pf_proj(const sxq_lm* lm, const QWeight& w, const float* x, const uint8_t* act, int T, float* y,
                    const float* bias, const float* res, bool exact, void* gemm_ws, hipStream_t s) {
     const int64_t n = w.n;
@@ -427,14 +427,7 @@ hipError_t pf_proj(const sxq_lm* lm, const QWeight& w, const float* x, const uin
         return e == hipSuccess ? launch_gemm_q4k(w, gemm_ws, T, y, n, bias, res, n, s) : e;
     }
     if (w.dtype != kQ4K && T >= kGemmQ80MinRows) return launch_gemm_q80(w, act, T, y, n, bias, res, n, s);
-    const size_t rowb = (size_t)(w.k / block_size(lm->vdt)) * act_block_bytes(lm->vdt);
-    for (int r0 = 0; r0 < T; r0 += 16) {
-        const int mm = T - r0 < 16 ? T - r0 : 16;
-        hipError_t e = launch_gemv(w, act + (size_t)r0 * rowb, mm, y + (int64_t)r0 * n, n, bias,
-                                   res ? res + (int64_t)r0 * n : nullptr, n, s);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    return launch_gemv(w, act, T, y, n, bias, res, n, s);
 }
 
 // Device buffers of one prefill of T tokens over n streams (offsets into lm->pf).

@@ -15,8 +15,21 @@ namespace sxq {
 // Activation quantization kernel: rows x [m, k] (row stride ldx floats) -> blocks.
 // One wave per 256-element chunk.  out_canon: canonical Candle blocks [m][k/bs];
 // otherwise the device layout ActQ8K/ActQ8_0 [m][k/bs].
-template <int VDT, bool CANON>
-__global__ __launch_bounds__(256) void k_quantize_act(const float* __restrict__ x, int64_t ldx, int m,
+// XT: float, or uint16_t for bf16 rows.  V: rows are aligned for the four-element load.
+template <bool V, typename XT>
+SXQ_DEV float4 act_load4(const XT* p) {
+    if constexpr (sizeof(XT) == 4) {
+        return *(const float4*)p;
+    } else {
+        ushort4 u;
+        if (V) u = *(const ushort4*)p;
+        else u = make_ushort4(p[0], p[1], p[2], p[3]);
+        return make_float4(__uint_as_float((uint32_t)u.x << 16), __uint_as_float((uint32_t)u.y << 16),
+                           __uint_as_float((uint32_t)u.z << 16), __uint_as_float((uint32_t)u.w << 16));
+    }
+}
+template <int VDT, bool CANON, typename XT = float, bool V = true>
+__global__ __launch_bounds__(256) void k_quantize_act(const XT* __restrict__ x, int64_t ldx, int m,
                                                       int k, void* __restrict__ out) {
     const int lane = threadIdx.x & 63;
     const int chunk = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -24,9 +37,9 @@ __global__ __launch_bounds__(256) void k_quantize_act(const float* __restrict__ 
     const int row = blockIdx.y;
     if (row >= m || chunk >= chunks_per_row) return;
     const int e0 = chunk * 256 + 4 * lane;
-    const float* xr = x + (int64_t)row * ldx;
+    const XT* xr = x + (int64_t)row * ldx;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (e0 < k) v = *(const float4*)(xr + e0);  // k is a multiple of 32, so 4 | k
+    if (e0 < k) v = act_load4<V>(xr + e0);  // k is a multiple of 32, so 4 | k
     if (VDT == kQ8K) {
         const int nb = k / 256;
         char* base = (char*)out + ((int64_t)row * nb + chunk) * (CANON ? sizeof(BlockQ8K) : sizeof(ActQ8K));
@@ -50,6 +63,22 @@ hipError_t launch_quantize_act(int vdt, bool canon, const float* x, int64_t ldx,
         if (canon) hipLaunchKernelGGL((k_quantize_act<kQ8_0, true>), grid, dim3(256), 0, s, x, ldx, m, k, out);
         else hipLaunchKernelGGL((k_quantize_act<kQ8_0, false>), grid, dim3(256), 0, s, x, ldx, m, k, out);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_quantize_act_bf16(int vdt, const uint16_t* x, int64_t ldx, int m, int k, void* out, hipStream_t s) {
+    const dim3 grid(((k + 255) / 256 + 3) / 4, m);
+    const bool vec = ((uintptr_t)x & 7) == 0 && ldx % 4 == 0;
+#define SXQ_QUANT_BF16(VDT, V) \
+    hipLaunchKernelGGL((k_quantize_act<VDT, false, uint16_t, V>), grid, dim3(256), 0, s, x, ldx, m, k, out)
+    if (vdt == kQ8K) {
+        if (vec) SXQ_QUANT_BF16(kQ8K, true);
+        else SXQ_QUANT_BF16(kQ8K, false);
+    } else {
+        if (vec) SXQ_QUANT_BF16(kQ8_0, true);
+        else SXQ_QUANT_BF16(kQ8_0, false);
+    }
+#undef SXQ_QUANT_BF16
     return hipGetLastError();
 }
 
