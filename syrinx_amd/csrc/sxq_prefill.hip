@@ -42,145 +42,199 @@ __global__ __launch_bounds__(64) void k_prefill_rope_kv(const float* __restrict_
     rope_store<HD>(rope_pair<HD>(ri, nw != nullptr, eps, inv_hd, lane), interleaved, dst, nullptr, lane);
 }
 
-constexpr int kPfRows = 64;  // query rows (tokens x heads of one KV group) per workgroup
-constexpr int kPfKeys = 64;  // key positions per LDS tile: 32 for each half of the waves
-
-// LDS row strides (floats): a lane's float4 reads of 16 consecutive keys, and the value reads
-// of 32 dims of two keys four apart, each hit every bank once.
-constexpr int pf_kstride(int hd) { return hd + 4; }
-constexpr int pf_vstride(int hd) { return hd + 8; }
-size_t prefill_attn_lds(int hd) {
-    const size_t tiles = sizeof(float) * (size_t)kPfKeys * (pf_kstride(hd) + pf_vstride(hd));
-    const size_t merge = sizeof(float) * 2 * 64 * (size_t)(hd / 2 + 2);  // two waves' accumulators, m and l
-    return tiles > merge ? tiles : merge;
-}
+constexpr int kPfRows = 64;    // query rows (tokens x heads of one KV group) per tile
+constexpr int kPfWgRows = 32;  // of them, rows per workgroup
+constexpr int kPfKeys = 32;    // key positions per LDS tile
+constexpr int kPfSStride = 36; // floats per row of scores: float4-aligned, the reads hit 64 banks
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-// One workgroup (256 threads) per (tile, KV group): a tile is up to kPfRows / G
-// consecutive prompt tokens of one stream (tile = {stream, first token row t0, count,
-// position p0 of token t0}); its rows are r = i * G + hh (token i, query head g * G + hh).
-// Everything is f32 on the f32 matrix cores (v_mfma_f32_32x32x2_f32), transposed so that a
-// row's softmax stays in its lane: wave w holds rows 32 (w & 1) .. +31 and takes the 32-key
-// halves w >> 1 of the tiles; lane (c, h) = (lane & 31, lane >> 5) owns row c.
-//   scores^T = K Q^T: result i of a lane is key 8 (i / 4) + 4 h + i % 4 of its row (the query
-//     row is in the lane's registers for the whole kernel; K's dims are taken in the order 8 u
-//     + 4 h + t, so that a lane reads float4s);
-//   out^T += V^T P^T: the probabilities are already the operand the product needs (MFMA i takes
-//     that key from half h), V comes from LDS a row of 32 dims at a time.
-// Each wave keeps an online softmax (running max m, sum l, rescaled accumulator) over its own
-// keys, masking keys past a row's own position; the two halves' results meet in LDS at the end.
-// Bound by the f32 matrix cores (64 cycles per 4096 flops): 1412 ragged tokens of 32 / 8 heads of
-// 128 in 196 us per layer, 226 tokens of 14 / 2 heads of 64 in 21.4 us; with the same tiles
-// on the VALU (a score per thread, four threads per row) 591 and 66 us.  Tiles are taken last
-// first: the last tokens of a prompt attend the most keys.
+// Exchanges lanes 32..63 of a with lanes 0..31 of b.
+SXQ_DEV void swap32(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+// Exchanges the odd 16-lane rows of a with the even ones of b (row 1 with 0, row 3 with 2).
+SXQ_DEV void swap16(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+
+// A wave's share of a 32-row tile of HD floats, straight to LDS: row r's 16-byte piece p goes
+// to slot p ^ (r & SW) of its row (SW = 15: reads of one element of 16 rows hit 64 banks).
+// off(r) is the byte offset of row r's data.
+template <int HD, int SW, typename F>
+SXQ_DEV void pf_tile_to_lds(__amdgpu_buffer_rsrc_t src, float* dst, int wave, int lane, F&& off) {
+    constexpr int PR = HD / 4, NI = 32 * PR / 256;  // pieces per row, loads per wave
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int at = (wave * NI + i) * 64, r = (at + lane) / PR, p = (at + lane) % PR;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)(dst + 4 * at), 16,
+                                                 off(r) + 16u * (uint32_t)(p ^ (r & SW)), 0, 0, 0);
+    }
+}
+
+// One workgroup (256 threads) per (tile, KV group, half of the tile's rows): a tile is up to
+// kPfRows / G consecutive prompt tokens of one stream (tile = {stream, first token row t0,
+// count, position p0 of token t0}); its rows are r = i * G + hh (token i, query head
+// g * G + hh).  Keys go through LDS 32 at a time, every row keeps an online softmax (running
+// max m, sum l, rescaled accumulator) and masks the keys past its own position.
+//
+// The arithmetic is that of one multiply and one add per term, each rounded, terms in order
+// (a score over the head dims, an output over the keys), whatever the split: the products
+// come from v_mfma_f32_16x16x1_4b_f32 with a zero addend (four outer products of a rank-1
+// update each: four head dims of 16 keys x 16 rows, or four keys of 16 dims x 16 rows), and
+// the VALU adds the four blocks in order.  So the VALU issues one operation per term in
+// place of two, and the matrix cores run beside it at half their rate.
+//   wave w: rows 16 (w & 1) .. +15; keys 16 (w >> 1) .. +15 of the tile for the scores,
+//   which meet in LDS, and head dims HD / 2 (w >> 1) .. for the outputs.  Lane (c, b) =
+//   (lane & 15, lane >> 4) supplies element c of block b and holds row c in the results.
+// K is read while V loads and V while the next K loads (direct to LDS, one buffer each).
+// SXQ_PF_MEASURED
 template <int HD>
-__global__ __launch_bounds__(256, 2) void k_prefill_attn(const float* __restrict__ q, const float* __restrict__ kc,
+__global__ __launch_bounds__(256, 3) void k_prefill_attn(const float* __restrict__ q, const float* __restrict__ kc,
                                                          const float* __restrict__ vc, const int4* __restrict__ tiles,
                                                          int nh, int nkv, int max_seq, int64_t kv_stream_stride,
                                                          float scale, float* __restrict__ ctx) {
-    extern __shared__ float4 smem4[];
-    constexpr int KS = pf_kstride(HD), VS = pf_vstride(HD), U = HD / 8, DG = HD / 32;
-    const int4 tl = tiles[gridDim.x - 1 - blockIdx.x];
+    constexpr int U = HD / 4, DT = HD / 32;  // head-dim quads; 16-dim tiles of a wave's outputs
+    __shared__ float kt[kPfKeys * HD];       // queries first, then key tiles
+    __shared__ float vt[kPfKeys * HD];
+    __shared__ float st[kPfWgRows * kPfSStride];
+    const int4 tl = tiles[gridDim.x - 1 - blockIdx.x];  // the last tokens attend the most keys
     const int s = tl.x, t0 = tl.y, cnt = tl.z, p0 = tl.w;
-    const int g = blockIdx.y, G = nh / nkv, R = cnt * G;
-    float* kt = (float*)smem4;      // [kPfKeys][KS]
-    float* vt = kt + kPfKeys * KS;  // [kPfKeys][VS]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c = lane & 31, h = lane >> 5, half = wave >> 1;
-    const int row = 32 * (wave & 1) + c;
-    const int rr = min(row, R - 1);  // rows past the tile compute on a copy and store nothing
-    const int64_t qoff = (int64_t)(t0 + rr / G) * nh * HD + (g * G + rr % G) * HD;
+    const int g = blockIdx.y, G = nh / nkv, R = cnt * G, r0 = kPfWgRows * blockIdx.z;
+    if (r0 >= R) return;  // uniform
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, b = lane >> 4, rg = wave & 1, hv = wave >> 1;
+    const int row = r0 + 16 * rg + c, rr = min(row, R - 1);  // rows past the tile: a copy, not stored
     const int qpos = p0 + rr / G;
-    float4 qv[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) qv[u] = *(const float4*)(q + qoff + 8 * u + 4 * h);
-    float m = -INFINITY, l = 0.0f;
-    v16f o[DG];
-#pragma unroll
-    for (int d = 0; d < DG; ++d) o[d] = v16f{};
+    const int kend = p0 + min(r0 + kPfWgRows - 1, R - 1) / G + 1;
+    const __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(q + ((int64_t)t0 * nh + g * G) * HD), (short)0, (int)((uint32_t)(((cnt - 1) * nh + G) * HD) * 4u), 0x00020000);
+    pf_tile_to_lds<HD, 15>(qrs, kt, wave, lane, [&](int r) {
+        const int i = min(r0 + r, R - 1);
+        return (uint32_t)((i / G) * nh + i % G) * (HD * 4u);
+    });
     const int64_t koff = (int64_t)s * kv_stream_stride + (int64_t)g * max_seq * HD;
-    const int kend = p0 + cnt;
+    const __amdgpu_buffer_rsrc_t krs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kc + koff), (short)0, (int)((uint32_t)kend * HD * 4u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t vrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vc + koff), (short)0, (int)((uint32_t)kend * HD * 4u), 0x00020000);
+    // keys past the last one load it again (their probabilities are zero)
+    auto load_k = [&](int j0) {
+        pf_tile_to_lds<HD, 15>(krs, kt, wave, lane, [&](int r) { return (uint32_t)min(j0 + r, kend - 1) * (HD * 4u); });
+    };
+    auto load_v = [&](int j0) {
+        pf_tile_to_lds<HD, 0>(vrs, vt, wave, lane, [&](int r) { return (uint32_t)min(j0 + r, kend - 1) * (HD * 4u); });
+    };
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    float qv[U];  // head dim 4 u + b of row c
+#pragma unroll
+    for (int u = 0; u < U; ++u) qv[u] = kt[(16 * rg + c) * HD + 4 * (u ^ c) + b];
+    lds_barrier();  // kt is free
+    load_k(0);
+    float m = -INFINITY, l = 0.0f;
+    float o[DT][4];
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[t][e] = 0.0f;
     for (int j0 = 0; j0 < kend; j0 += kPfKeys) {
-        lds_barrier();  // the previous tile is no longer read
-        for (int e = tid; e < kPfKeys * (HD / 4); e += 256) {
-            const int key = e / (HD / 4), d = 4 * (e % (HD / 4));
-            float4 kv = make_float4(0.f, 0.f, 0.f, 0.f), vv = kv;
-            if (j0 + key < kend) {
-                kv = *(const float4*)(kc + koff + (int64_t)(j0 + key) * HD + d);
-                vv = *(const float4*)(vc + koff + (int64_t)(j0 + key) * HD + d);
-            }
-            *(float4*)(kt + key * KS + d) = kv;
-            *(float4*)(vt + key * VS + d) = vv;
-        }
-        lds_barrier();
-        const int jb = j0 + 32 * half;  // this wave's first key
-        if (jb >= kend) continue;       // uniform per wave; every wave reaches each barrier
-        v16f sc = v16f{};
-        const float* kr = kt + (32 * half + c) * KS + 4 * h;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();  // the keys are here; the previous values and scores are no longer read
+        load_v(j0);
+        float4 sc4 = make_float4(0.f, 0.f, 0.f, 0.f);  // keys 16 hv + 4 b + (0..3) of row c
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const float4 kv = *(const float4*)(kr + 8 * u);
-            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qv[u].x, sc, 0, 0, 0);
-            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qv[u].y, sc, 0, 0, 0);
-            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qv[u].z, sc, 0, 0, 0);
-            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qv[u].w, sc, 0, 0, 0);
-        }
-        float bm = -INFINITY;
+            const v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(kt[(16 * hv + c) * HD + 4 * (u ^ c) + b], qv[u], v16f{}, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int j = jb + 8 * (i >> 2) + 4 * h + (i & 3);
-            sc[i] = j <= qpos ? sc[i] * scale + 0.0f : -INFINITY;
-            bm = fmaxf(bm, sc[i]);
+            for (int k = 0; k < 4; ++k) {
+                sc4.x += d[4 * k];
+                sc4.y += d[4 * k + 1];
+                sc4.z += d[4 * k + 2];
+                sc4.w += d[4 * k + 3];
+            }
         }
-        bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
-        const float mn = fmaxf(m, bm);
+        *(float4*)(st + (16 * rg + c) * kPfSStride + 16 * hv + 4 * b) = sc4;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();  // the scores and values are here; the keys are no longer read
+        if (j0 + kPfKeys < kend) load_k(j0 + kPfKeys);
+        float p[8], bm = -INFINITY;  // key 4 i + b of row c
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float v = st[(16 * rg + c) * kPfSStride + 4 * i + b];
+            p[i] = j0 + 4 * i + b <= qpos ? v * scale + 0.0f : -INFINITY;
+            bm = fmaxf(bm, p[i]);
+        }
+        float x = bm, y = bm;
+        swap16(x, y);
+        bm = fmaxf(x, y);
+        x = y = bm;
+        swap32(x, y);
+        const float mn = fmaxf(m, fmaxf(x, y));
         const float corr = mn == -INFINITY ? 1.0f : expf(m - mn);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) p[i] = p[i] == -INFINITY ? 0.0f : expf(p[i] - mn);
+        // keys 8 b .. 8 b + 7 summed in order by row b of lanes, then the four sums in pairs
         float ps = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            sc[i] = sc[i] == -INFINITY ? 0.0f : expf(sc[i] - mn);
-            ps += sc[i];
+        for (int h = 0; h < 2; ++h) {
+            float a0 = p[h], a1 = p[2 + h], a2 = p[4 + h], a3 = p[6 + h];
+            swap32(a0, a2);
+            swap32(a1, a3);
+            swap16(a0, a1);
+            swap16(a2, a3);
+            ps += a0;
+            ps += a1;
+            ps += a2;
+            ps += a3;
         }
-        ps += __shfl_xor(ps, 32, 64);
+        x = y = ps;
+        swap16(x, y);
+        ps = x + y;
+        x = y = ps;
+        swap32(x, y);
+        ps = x + y;
         l = l * corr + ps;
         m = mn;
-        const float* vr = vt + (32 * half + 4 * h) * VS + c;
 #pragma unroll
-        for (int d = 0; d < DG; ++d) {
+        for (int t = 0; t < DT; ++t)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) o[d][i] *= corr;
+            for (int e = 0; e < 4; ++e) o[t][e] *= corr;
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
-                o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[(8 * (i >> 2) + (i & 3)) * VS + 32 * d], sc[i], o[d], 0, 0, 0);
+        for (int i = 0; i < 8; ++i) {
+            float vv[DT];
+            const float* vr = vt + (4 * i + b) * HD + (HD / 2) * hv + DT * c;
+            if constexpr (DT == 4) {
+                const float4 f = *(const float4*)vr;
+                vv[0] = f.x, vv[1] = f.y, vv[2] = f.z, vv[3] = f.w;
+            } else {
+                const float2 f = *(const float2*)vr;
+                vv[0] = f.x, vv[1] = f.y;
+            }
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                const v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(vv[t], p[i], v16f{}, 0, 0, 0);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[t][e] += d[4 * k + e];
+            }
         }
     }
-    // the second half's waves hand their rows to the first half's
-    lds_barrier();
-    float* ex = (float*)smem4 + (wave & 1) * 64 * (HD / 2 + 2);
-    if (half == 1) {
+    if (row >= R) return;
+    // o[t][e] is head dim HD / 2 hv + DT (4 b + e) + t: 4 DT consecutive dims a lane
+    float* out = ctx + ((int64_t)(t0 + rr / G) * nh + g * G + rr % G) * HD + (HD / 2) * hv + 4 * DT * b;
+    float f[4 * DT];
 #pragma unroll
-        for (int d = 0; d < DG; ++d)
+    for (int t = 0; t < DT; ++t)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) ex[(16 * d + i) * 64 + lane] = o[d][i];
-        ex[(HD / 2) * 64 + lane] = m;
-        ex[(HD / 2 + 1) * 64 + lane] = l;
-    }
-    lds_barrier();
-    if (half == 1 || row >= R) return;
-    const float m1 = ex[(HD / 2) * 64 + lane], l1 = ex[(HD / 2 + 1) * 64 + lane];
-    const float mn = fmaxf(m, m1);
-    const float c0 = mn == -INFINITY ? 1.0f : expf(m - mn), c1 = mn == -INFINITY ? 1.0f : expf(m1 - mn);
-    const float lt = l * c0 + l1 * c1;
+        for (int e = 0; e < 4; ++e) f[DT * e + t] = o[t][e] / l;
 #pragma unroll
-    for (int d = 0; d < DG; ++d)
-#pragma unroll
-        for (int i = 0; i < 16; i += 4) {
-            float v[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) v[t] = (o[d][i + t] * c0 + ex[(16 * d + i + t) * 64 + lane] * c1) / lt;
-            *(float4*)(ctx + qoff + 32 * d + 2 * i + 4 * h) = make_float4(v[0], v[1], v[2], v[3]);
-        }
+    for (int i = 0; i < DT; ++i) *(float4*)(out + 4 * i) = make_float4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
 }
 
 // One thread per token t (and per tile index): stream-major order, stream s's tokens at
@@ -252,21 +306,14 @@ hipError_t launch_prefill_attn(const float* q, const float* kc, const float* vc,
                                int nkv, int hd, int max_seq, int64_t kv_stream_stride, float* ctx, hipStream_t s) {
     if (!prefill_attn_supported(nh, nkv, hd)) return hipErrorInvalidValue;
     if (n_tiles == 0) return hipSuccess;
-    const size_t lds = prefill_attn_lds(hd);
     const float scale = (float)(1.0 / sqrt((double)hd));
-    if (hd == 128) {
-        static const hipError_t a = hipFuncSetAttribute((const void*)k_prefill_attn<128>,
-                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefill_attn_lds(128));
-        if (a != hipSuccess) return a;
-        hipLaunchKernelGGL(k_prefill_attn<128>, dim3(n_tiles, nkv), dim3(256), lds, s, q, kc, vc, (const int4*)tiles,
-                           nh, nkv, max_seq, kv_stream_stride, scale, ctx);
-    } else {
-        static const hipError_t a = hipFuncSetAttribute((const void*)k_prefill_attn<64>,
-                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefill_attn_lds(64));
-        if (a != hipSuccess) return a;
-        hipLaunchKernelGGL(k_prefill_attn<64>, dim3(n_tiles, nkv), dim3(256), lds, s, q, kc, vc, (const int4*)tiles,
-                           nh, nkv, max_seq, kv_stream_stride, scale, ctx);
-    }
+    const dim3 grid(n_tiles, nkv, kPfRows / kPfWgRows);
+    if (hd == 128)
+        hipLaunchKernelGGL(k_prefill_attn<128>, grid, dim3(256), 0, s, q, kc, vc, (const int4*)tiles, nh, nkv, max_seq,
+                           kv_stream_stride, scale, ctx);
+    else
+        hipLaunchKernelGGL(k_prefill_attn<64>, grid, dim3(256), 0, s, q, kc, vc, (const int4*)tiles, nh, nkv, max_seq,
+                           kv_stream_stride, scale, ctx);
     return hipGetLastError();
 }
 
