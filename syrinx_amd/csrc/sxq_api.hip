@@ -65,6 +65,7 @@ struct WorkspaceLease {
     uint8_t* ptr = nullptr;
     hipError_t err = hipSuccess;
     WorkspaceLease(int dev, size_t need, hipStream_t st) : s(st) {
+        if (need == 0) return;  // nothing to hold: no turn to take
         if (dev < 0 || dev >= 64) { err = hipErrorInvalidDevice; return; }
         w = &g_ws[dev];
         w->mu.lock();
@@ -331,14 +332,16 @@ sxq_status plan_forward(const sxq_qmm* q, const int64_t* shape, int ndim, const 
     // for Candle's integer vec-dot (the GEMV, 16 rows at a time).
     const bool q80 = q->w.dtype == kQ8_0 || q->w.dtype == kQ4_0;
     p->gemm = q80 ? m >= kGemmQ80MinRows : (m >= kGemmMinRows && !(flags & SXQ_BIT_EXACT));
-    p->ws = m == 0 ? 0
-                   : up256(p->gemm && !q80 ? gemm_q4k_workspace(q->w.n, (int)m, q->w.k)
-                                           : (size_t)m * (size_t)p->nbv * act_block_bytes(p->vdt));
+    // one row that its GEMV quantizes needs none
+    const bool row = m == 1 && fused_quant(q->w);
+    p->ws = m == 0 || row ? 0
+                          : up256(p->gemm && !q80 ? gemm_q4k_workspace(q->w.n, (int)m, q->w.k)
+                                                  : (size_t)m * (size_t)p->nbv * act_block_bytes(p->vdt));
     // bf16 input: the quantizer reads it (an exact widening in registers: no launch and no f32
     // copy of x).  The f16 GEMM and the one-row GEMV that quantizes in its prologue take f32
     // rows: widened to f32 at the workspace's end, then the f32 forward.
     p->bf16 = (flags & SXQ_BF16_INPUT) && m > 0;
-    const bool f32_rows = (p->gemm && !q80) || (m == 1 && fused_quant(q->w));
+    const bool f32_rows = (p->gemm && !q80) || row;
     p->xconv = p->bf16 && f32_rows ? up256((size_t)m * (size_t)q->w.k * 4) : 0;
     p->ws += p->xconv;
     return SXQ_OK;

@@ -131,3 +131,32 @@ def test_prefill_attention_tiles(cuda, hd, G, nkv):
                     err = (got[at:at + c, g * G + h] - want).abs().max()
                     assert err <= tol, f"counts {counts} stream {s} head {g * G + h}: {float(err):.3g} > {float(tol):.3g}"
             at += c
+
+
+@pytest.mark.parametrize("dt,k", [(G.Q4K, 512), (G.Q8_0, 896), (G.Q4_0, 320)])
+@pytest.mark.parametrize("m", [1, 5, 70])
+def test_forward_workspaces(cuda, dt, k, m):
+    """The forward's workspace per call: calls that alternate between streams, and a captured
+    call replayed between eager ones (one row of Q8_0 / Q4_0 needs no workspace)."""
+    gen = torch.Generator(device=cuda).manual_seed(k + m)
+    qmm = QMatMul.from_qtensor(QTensor.quantize(torch.randn(300, k, generator=gen, device=cuda) * 0.02, dt))
+    xs = [torch.randn(m, k, generator=gen, device=cuda) for _ in range(8)]
+    want = [qmm.forward(x).clone() for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(device=cuda) for _ in range(2)]
+    got = []
+    for i, x in enumerate(xs):
+        with torch.cuda.stream(streams[i % 2]):
+            got.append(qmm.forward(x))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    xin = xs[0].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = qmm.forward(xin)
+    for x, w in zip(xs[:4], want):
+        xin.copy_(x)
+        graph.replay()
+        eager = qmm.forward(xs[5])
+        torch.cuda.synchronize()
+        assert torch.equal(y, w) and torch.equal(eager, want[5])
