@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "sxq_kernels.h"
+#include "sxq_quant_dev.h"
 #include "sxq_sync_dev.h"
 
 namespace sxq {
@@ -113,14 +114,26 @@ __global__ __launch_bounds__(256) void k_x_to_f16_perm(const float* __restrict__
     }
 }
 
-// The same conversion in one pass over x, for rows of k <= 1024 * V4 elements: the row is
+// The same conversion in one pass, for rows of k <= 1024 * V4 elements: the row is
 // loaded once (every thread's V4 float4 loads issued together), its max |x| reduced while
 // it goes to LDS, and the f16 positions gathered from LDS -- thread t writes the 16-byte
 // chunks t, t + 256, ... of the row (chunk c: block c / 32, positions 8 (c mod 32) .. + 7),
 // so the row's writes are contiguous.  The bits are k_x_to_f16_perm's.
-template <int V4>
+//
+// SRC says what the row is: kSrcRows x itself; kSrcNorm the RMSNorm of x's row with weights
+// w; kSrcSilu silu(g) * u of x's row [gate (k) | up (k)].  A prompt's projections take their
+// operand from these directly: no f32 row goes through memory (copy receives one if it is not
+// null) and nothing is quantized that the f16 product does not read.  The values are those of
+// k_rmsnorm_quant and k_silu_mul_quant bit for bit: the sum of squares is theirs, float4 i of
+// the row belonging to thread i mod 1024 of that kernel.  Bound by memory: 1412 rows
+// of silu(g) * u at k = 9728 in 37 us (165 MB: 4.4 TB/s) against 65 + 14 for the quantizing
+// kernel and the conversion of its f32 rows; of the RMSNorm at k = 2560 in 9.4 us against 39 + 6.
+constexpr int kSrcRows = 0, kSrcNorm = 1, kSrcSilu = 2;
+template <int V4, int SRC>
 __global__ __launch_bounds__(256) void k_x_to_f16_perm1(const float* __restrict__ x, int64_t ldx, int m, int k,
-                                                        _Float16* __restrict__ xh, float* __restrict__ rs) {
+                                                        _Float16* __restrict__ xh, float* __restrict__ rs,
+                                                        const float* __restrict__ w, float inv_n, float eps,
+                                                        float* __restrict__ copy) {
     extern __shared__ float4 rowbuf[];  // the row, k floats
     __shared__ float wmax[4];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -128,18 +141,61 @@ __global__ __launch_bounds__(256) void k_x_to_f16_perm1(const float* __restrict_
     const int64_t r = blockIdx.x;
     const bool live = r < m;
     const float4* xr = (const float4*)(x + r * ldx);
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 v[V4];
 #pragma unroll
     for (int j = 0; j < V4; ++j) {
         const int i = tid + 256 * j;
-        v[j] = live && i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+        v[j] = live && i < n4 ? xr[i] : zero;
+    }
+    if constexpr (SRC == kSrcNorm) {
+        __shared__ float red[16];
+        float ss[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < V4; ++j) {
+            ss[j & 3] += v[j].x * v[j].x;
+            ss[j & 3] += v[j].y * v[j].y;
+            ss[j & 3] += v[j].z * v[j].z;
+            ss[j & 3] += v[j].w * v[j].w;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            ss[q] = wave_sum_rows(ss[q]);
+            if (lane == 0) red[wave + 4 * q] = ss[q];
+        }
+        lds_barrier();
+        const float var = rmsnorm_tree_16(red) * inv_n + 0.0f;
+        const float den = sqrtf(var * 1.0f + eps);
+        if (live) {
+#pragma unroll
+            for (int j = 0; j < V4; ++j) {
+                const int i = tid + 256 * j;
+                if (i < n4) {
+                    const float4 wv = ((const float4*)w)[i];
+                    v[j] = make_float4((v[j].x / den) * wv.x, (v[j].y / den) * wv.y, (v[j].z / den) * wv.z,
+                                       (v[j].w / den) * wv.w);
+                }
+            }
+        }
+    }
+    if constexpr (SRC == kSrcSilu) {
+        auto silu = [](float g, float u) { return (g / (1.0f + expf(-g))) * u; };
+#pragma unroll
+        for (int j = 0; j < V4; ++j) {
+            const int i = tid + 256 * j;
+            const float4 u = live && i < n4 ? xr[n4 + i] : zero;
+            v[j] = make_float4(silu(v[j].x, u.x), silu(v[j].y, u.y), silu(v[j].z, u.z), silu(v[j].w, u.w));
+        }
     }
     float amax = 0.0f;
 #pragma unroll
     for (int j = 0; j < V4; ++j) {
         const int i = tid + 256 * j;
         amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
-        if (i < n4) rowbuf[i] = v[j];
+        if (i < n4) {
+            rowbuf[i] = v[j];
+            if (SRC != kSrcRows && copy && live) ((float4*)(copy + r * k))[i] = v[j];
+        }
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
@@ -598,19 +654,43 @@ size_t gemm_q4k_workspace(int64_t n, int m, int64_t k) {
     return p.xh_bytes + p.rs_bytes + p.part_bytes;
 }
 
-hipError_t launch_gemm_q4k_prep(const float* x, int64_t ldx, int m, int64_t n, int k, void* ws, hipStream_t s) {
+// The one-pass preparation of a row source (m rows of k <= kPrepMaxK elements).
+template <int SRC>
+static void prep_rows(const float* x, int64_t ldx, int m, int64_t n, int k, void* ws, const float* w, float eps,
+                      float* copy, hipStream_t s) {
     const GemmPlan p = gemm_plan(n, m, k);
-    const int rows = gemm_xh_rows(m);
     _Float16* xh = (_Float16*)ws;
     float* rs = (float*)((uint8_t*)ws + p.xh_bytes);
-    const bool two_pass = getenv("SXQ_X2F16_TWO_PASS") != nullptr;  // A/B: the two-pass conversion
+    const dim3 grid((unsigned)gemm_xh_rows(m)), block(256);
     const size_t row_lds = (size_t)k * sizeof(float);
-    if (!two_pass && k <= 4096)
-        hipLaunchKernelGGL(k_x_to_f16_perm1<4>, dim3((unsigned)rows), dim3(256), row_lds, s, x, ldx, m, k, xh, rs);
-    else if (!two_pass && k <= 12288)
-        hipLaunchKernelGGL(k_x_to_f16_perm1<12>, dim3((unsigned)rows), dim3(256), row_lds, s, x, ldx, m, k, xh, rs);
+    const float inv_n = (float)(1.0 / (double)k);
+    if (k <= 4096)
+        hipLaunchKernelGGL((k_x_to_f16_perm1<4, SRC>), grid, block, row_lds, s, x, ldx, m, k, xh, rs, w, inv_n, eps, copy);
     else
-        hipLaunchKernelGGL(k_x_to_f16_perm, dim3((unsigned)rows), dim3(256), 0, s, x, ldx, m, k, xh, rs);
+        hipLaunchKernelGGL((k_x_to_f16_perm1<12, SRC>), grid, block, row_lds, s, x, ldx, m, k, xh, rs, w, inv_n, eps, copy);
+}
+
+hipError_t launch_gemm_q4k_prep(const float* x, int64_t ldx, int m, int64_t n, int k, void* ws, hipStream_t s) {
+    const bool two_pass = getenv("SXQ_X2F16_TWO_PASS") != nullptr;  // A/B: the two-pass conversion
+    if (!two_pass && k <= kPrepMaxK) {
+        prep_rows<kSrcRows>(x, ldx, m, n, k, ws, nullptr, 0.0f, nullptr, s);
+    } else {
+        const GemmPlan p = gemm_plan(n, m, k);
+        hipLaunchKernelGGL(k_x_to_f16_perm, dim3((unsigned)gemm_xh_rows(m)), dim3(256), 0, s, x, ldx, m, k,
+                           (_Float16*)ws, (float*)((uint8_t*)ws + p.xh_bytes));
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm_q4k_prep_norm(const NormIn& ni, int m, int64_t n, int k, void* ws, hipStream_t s) {
+    if (k > kPrepMaxK) return hipErrorInvalidValue;
+    prep_rows<kSrcNorm>(ni.x, k, m, n, k, ws, ni.w, ni.eps, ni.normed, s);
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm_q4k_prep_silu(const float* gu, int m, int64_t n, int k, void* ws, float* copy, hipStream_t s) {
+    if (k > kPrepMaxK) return hipErrorInvalidValue;
+    prep_rows<kSrcSilu>(gu, 2 * (int64_t)k, m, n, k, ws, nullptr, 0.0f, copy, s);
     return hipGetLastError();
 }
 

@@ -98,6 +98,12 @@ constexpr int kGemmMinRows = 64;  // QMatMul::forward uses the Q4_K GEMM from th
 constexpr int kGemmQ80MinRows = 5;  // ... and the Q8_0 / Q4_0 matrix-core kernels (below: the GEMV)
 size_t gemm_q4k_workspace(int64_t n, int m, int64_t k);
 hipError_t launch_gemm_q4k_prep(const float* x, int64_t ldx, int m, int64_t n, int k, void* ws, hipStream_t s);
+// The same workspace from rows that are still to be computed, for k <= kPrepMaxK: the RMSNorm
+// of ni.x [m][k] (the f32 rows to ni.normed if it is not null), or silu(gate) * up of gu
+// [m][2k] (to copy if it is not null).  The values of k_rmsnorm_quant and k_silu_mul_quant.
+constexpr int kPrepMaxK = 12288;
+hipError_t launch_gemm_q4k_prep_norm(const NormIn& ni, int m, int64_t n, int k, void* ws, hipStream_t s);
+hipError_t launch_gemm_q4k_prep_silu(const float* gu, int m, int64_t n, int k, void* ws, float* copy, hipStream_t s);
 hipError_t launch_gemm_q4k(const QWeight& w, const void* ws, int m, float* y, int64_t ldy, const float* bias,
                            const float* res, int64_t ldr, hipStream_t s);
 

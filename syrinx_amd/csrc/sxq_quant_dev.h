@@ -66,14 +66,17 @@ SXQ_DEV float wave_max_rows(float v) {
 // is the RMSNorm sum of squares of every kernel here (fused GEMV prologue and the
 // standalone RMSNorm), so they agree bit for bit.  `red`: 16 floats of LDS.  Every
 // thread of the workgroup must call it (it synchronises, on LDS only).
-SXQ_DEV float rmsnorm_sumsq_1024(float ss, float* red) {
-    ss = wave_sum_rows(ss);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    lds_barrier();
+SXQ_DEV float rmsnorm_tree_16(const float* red) {
     float t[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) t[i] = red[2 * i] + red[2 * i + 1];
     return ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+}
+SXQ_DEV float rmsnorm_sumsq_1024(float ss, float* red) {
+    ss = wave_sum_rows(ss);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    lds_barrier();
+    return rmsnorm_tree_16(red);
 }
 
 // Round half away from zero (Rust's f32::round) of a finite or NaN value.

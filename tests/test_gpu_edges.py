@@ -160,3 +160,35 @@ def test_forward_workspaces(cuda, dt, k, m):
         eager = qmm.forward(xs[5])
         torch.cuda.synchronize()
         assert torch.equal(y, w) and torch.equal(eager, want[5])
+
+
+@pytest.mark.parametrize("dim,inter,T", [(256, 512, 64), (1280, 4352, 65), (4352, 256, 257)])
+def test_prefill_f16_sources(cuda, dim, inter, T):
+    """The f16 prompt path, whose projections prepare their operand from the RMSNorm and the
+    SwiGLU: the rows a trace records against 64 bits, and the same logits without a trace."""
+    from syrinx_amd.decoder import ATTN_NORM, FFN_NORM, DecoderConfig, DecoderLM
+    cfg = DecoderConfig(n_layers=1, dim=dim, n_heads=4, n_kv_heads=2, head_dim=64, intermediate=inter, vocab=64,
+                        max_seq=T, max_batch=1, weight_dtype=int(G.Q4K), tied_embedding=0, qk_norm=0)
+    lm = DecoderLM(cfg, device=cuda)
+    lm.init_random(seed=7, std=0.05)
+    gen = torch.Generator(device=cuda).manual_seed(dim + T)
+    w = {n: 1 + 0.2 * torch.randn(dim, generator=gen, device=cuda) for n in (ATTN_NORM, FFN_NORM)}
+    for n, v in w.items():
+        lm.set_vector(0, n, v)
+    x = torch.randn(T, dim, generator=gen, device=cuda) * torch.logspace(-3, 3, T, device=cuda)[:, None]
+    logits, _, hidden, tr = lm.prefill(embeds=[x], all_logits=True, trace=True)
+    lm.reset(1)
+    again = lm.prefill(embeds=[x], all_logits=True)
+    assert torch.equal(again[0], logits) and torch.equal(again[2], hidden)
+    layer = {k: torch.from_numpy(v).to(cuda).double().view(T, -1) for k, v in tr["layers"][0].items()}
+
+    def norm(h, n):
+        return h / (h.pow(2).mean(-1, keepdim=True) + cfg.norm_eps).sqrt() * w[n].double()
+
+    gate, up = layer["gu"].split(inter, -1)
+    for name, got, want in [("hn_attn", layer["hn_attn"], norm(x.double(), ATTN_NORM)),
+                            ("hn_ffn", layer["hn_ffn"], norm(layer["h_mid"], FFN_NORM)),
+                            ("act", layer["act"], torch.nn.functional.silu(gate) * up)]:
+        # a few roundings of f32 (the sum of squares is a tree: its error grows with its depth)
+        err = ((got - want).abs() / want.abs().clamp_min(1e-30)).max()
+        assert err < 32 * 2.0 ** -24, f"{name}: relative error {float(err):.3g}"
