@@ -42,10 +42,7 @@ __global__ __launch_bounds__(64) void k_prefill_rope_kv(const float* __restrict_
     rope_store<HD>(rope_pair<HD>(ri, nw != nullptr, eps, inv_hd, lane), interleaved, dst, nullptr, lane);
 }
 
-constexpr int kPfRows = 64;    // query rows (tokens x heads of one KV group) per tile
-constexpr int kPfWgRows = 32;  // of them, rows per workgroup
-constexpr int kPfKeys = 32;    // key positions per LDS tile
-constexpr int kPfSStride = 36; // floats per row of scores: float4-aligned, the reads hit 64 banks
+constexpr int kPfRows = 64;  // query rows (tokens x heads of one KV group) per tile
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 
@@ -62,25 +59,24 @@ SXQ_DEV void swap16(float& a, float& b) {
     b = __uint_as_float(r[1]);
 }
 
-// A wave's share of a 32-row tile of HD floats, straight to LDS: row r's 16-byte piece p goes
-// to slot p ^ (r & SW) of its row (SW = 15: reads of one element of 16 rows hit 64 banks).
-// off(r) is the byte offset of row r's data.
-template <int HD, int SW, typename F>
-SXQ_DEV void pf_tile_to_lds(__amdgpu_buffer_rsrc_t src, float* dst, int wave, int lane, F&& off) {
-    constexpr int PR = HD / 4, NI = 32 * PR / 256;  // pieces per row, loads per wave
+// A wave's share of a tile of ROWS rows of HD floats, straight to LDS: row r's 16-byte piece
+// p goes to slot p ^ sw(r) of its row.  off(r) is the byte offset of row r's data.
+template <int HD, int ROWS, typename O, typename S>
+SXQ_DEV void pf_tile_to_lds(__amdgpu_buffer_rsrc_t src, float* dst, int wave, int lane, O&& off, S&& sw) {
+    constexpr int PR = HD / 4, NI = ROWS * PR / 256;  // pieces per row, loads per wave
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int at = (wave * NI + i) * 64, r = (at + lane) / PR, p = (at + lane) % PR;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)(dst + 4 * at), 16,
-                                                 off(r) + 16u * (uint32_t)(p ^ (r & SW)), 0, 0, 0);
+                                                 off(r) + 16u * (uint32_t)(p ^ sw(r)), 0, 0, 0);
     }
 }
 
-// One workgroup (256 threads) per (tile, KV group, half of the tile's rows): a tile is up to
+// One workgroup (256 threads) per (tile, KV group, share of the tile's rows): a tile is up to
 // kPfRows / G consecutive prompt tokens of one stream (tile = {stream, first token row t0,
 // count, position p0 of token t0}); its rows are r = i * G + hh (token i, query head
-// g * G + hh).  Keys go through LDS 32 at a time, every row keeps an online softmax (running
-// max m, sum l, rescaled accumulator) and masks the keys past its own position.
+// g * G + hh).  Keys go through LDS 16 NP at a time, every row keeps an online softmax (running
+// max m, sum l, rescaled accumulator) over blocks of 32 and masks the keys past its own position.
 //
 // The arithmetic is that of one multiply and one add per term, each rounded, terms in order
 // (a score over the head dims, an output over the keys), whatever the split: the products
@@ -88,35 +84,49 @@ SXQ_DEV void pf_tile_to_lds(__amdgpu_buffer_rsrc_t src, float* dst, int wave, in
 // update each: four head dims of 16 keys x 16 rows, or four keys of 16 dims x 16 rows), and
 // the VALU adds the four blocks in order.  So the VALU issues one operation per term in
 // place of two, and the matrix cores run beside it at half their rate.
-//   wave w: rows 16 (w & 1) .. +15; keys 16 (w >> 1) .. +15 of the tile for the scores,
-//   which meet in LDS, and head dims HD / 2 (w >> 1) .. for the outputs.  Lane (c, b) =
-//   (lane & 15, lane >> 4) supplies element c of block b and holds row c in the results.
+//   wave w: rows 16 (w / NP) .. +15 of the workgroup's 64 / NP; keys 16 (w % NP) .. +15 of the
+//   tile for the scores, which meet in LDS, and head dims HD / NP (w % NP) .. for the outputs.
+//   Lane (c, b) = (lane & 15, lane >> 4) supplies element c of block b and holds row c in the
+//   results.
 // K is read while V loads and V while the next K loads (direct to LDS, one buffer each).
-// SXQ_PF_MEASURED
-template <int HD>
+// Bound by VALU issue: 1412 ragged tokens of 32 / 8 heads of 128 in 242 us per layer (591 with
+// both operations on the VALU, a score per thread and four threads per row; 104 M VALU
+// instructions, 170 us of issue), 226 tokens of 14 / 2 heads of 64 in 16.4 us (66).
+template <int HD, int NP>
 __global__ __launch_bounds__(256, 3) void k_prefill_attn(const float* __restrict__ q, const float* __restrict__ kc,
                                                          const float* __restrict__ vc, const int4* __restrict__ tiles,
                                                          int nh, int nkv, int max_seq, int64_t kv_stream_stride,
                                                          float scale, float* __restrict__ ctx) {
-    constexpr int U = HD / 4, DT = HD / 32;  // head-dim quads; 16-dim tiles of a wave's outputs
-    __shared__ float kt[kPfKeys * HD];       // queries first, then key tiles
-    __shared__ float vt[kPfKeys * HD];
-    __shared__ float st[kPfWgRows * kPfSStride];
-    const int4 tl = tiles[gridDim.x - 1 - blockIdx.x];  // the last tokens attend the most keys
+    constexpr int KT = 16 * NP, RW = 64 / NP;     // keys and rows per workgroup
+    constexpr int U = HD / 4, DW = HD / NP, DT = DW / 16;  // head-dim quads; dims of a wave's outputs, in 16s
+    constexpr int SS = KT + 4;  // floats per row of scores: float4-aligned, the reads hit 64 banks
+    __shared__ float kt[KT * HD];  // queries first, then key tiles
+    __shared__ float vt[KT * HD];
+    __shared__ float st[RW * SS];
+    // workgroups in the order of their tiles, which end latest first (k_prefill_tables): a tile
+    // at 1024 keys takes about half of the launch, and starting one of them late left a third of
+    // the CUs' time idle (310 us with each head's tiles in turn)
+    constexpr int NZ = kPfRows / RW;
+    const int sub = blockIdx.x % (nkv * NZ);
+    const int4 tl = tiles[blockIdx.x / (nkv * NZ)];
     const int s = tl.x, t0 = tl.y, cnt = tl.z, p0 = tl.w;
-    const int g = blockIdx.y, G = nh / nkv, R = cnt * G, r0 = kPfWgRows * blockIdx.z;
+    const int g = sub / NZ, G = nh / nkv, R = cnt * G, r0 = RW * (sub % NZ);
     if (r0 >= R) return;  // uniform
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int c = lane & 15, b = lane >> 4, rg = wave & 1, hv = wave >> 1;
+    const int c = lane & 15, b = lane >> 4, rg = wave / NP, part = wave % NP;
     const int row = r0 + 16 * rg + c, rr = min(row, R - 1);  // rows past the tile: a copy, not stored
     const int qpos = p0 + rr / G;
-    const int kend = p0 + min(r0 + kPfWgRows - 1, R - 1) / G + 1;
+    const int kend = p0 + min(r0 + RW - 1, R - 1) / G + 1;
+    // reads of one element of 16 rows (keys, queries), or of DT elements of 16 lanes in 4 rows
+    // (values), hit every bank
+    auto ksw = [](int r) { return r & 15; };
+    auto vsw = [](int r) { return DT >= 4 ? 0 : 4 * DT * (r & (4 / DT - 1)); };
     const __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(q + ((int64_t)t0 * nh + g * G) * HD), (short)0, (int)((uint32_t)(((cnt - 1) * nh + G) * HD) * 4u), 0x00020000);
-    pf_tile_to_lds<HD, 15>(qrs, kt, wave, lane, [&](int r) {
+    pf_tile_to_lds<HD, RW>(qrs, kt, wave, lane, [&](int r) {
         const int i = min(r0 + r, R - 1);
         return (uint32_t)((i / G) * nh + i % G) * (HD * 4u);
-    });
+    }, ksw);
     const int64_t koff = (int64_t)s * kv_stream_stride + (int64_t)g * max_seq * HD;
     const __amdgpu_buffer_rsrc_t krs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kc + koff), (short)0, (int)((uint32_t)kend * HD * 4u), 0x00020000);
@@ -124,10 +134,10 @@ __global__ __launch_bounds__(256, 3) void k_prefill_attn(const float* __restrict
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vc + koff), (short)0, (int)((uint32_t)kend * HD * 4u), 0x00020000);
     // keys past the last one load it again (their probabilities are zero)
     auto load_k = [&](int j0) {
-        pf_tile_to_lds<HD, 15>(krs, kt, wave, lane, [&](int r) { return (uint32_t)min(j0 + r, kend - 1) * (HD * 4u); });
+        pf_tile_to_lds<HD, KT>(krs, kt, wave, lane, [&](int r) { return (uint32_t)min(j0 + r, kend - 1) * (HD * 4u); }, ksw);
     };
     auto load_v = [&](int j0) {
-        pf_tile_to_lds<HD, 0>(vrs, vt, wave, lane, [&](int r) { return (uint32_t)min(j0 + r, kend - 1) * (HD * 4u); });
+        pf_tile_to_lds<HD, KT>(vrs, vt, wave, lane, [&](int r) { return (uint32_t)min(j0 + r, kend - 1) * (HD * 4u); }, vsw);
     };
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
@@ -142,92 +152,101 @@ __global__ __launch_bounds__(256, 3) void k_prefill_attn(const float* __restrict
     for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[t][e] = 0.0f;
-    for (int j0 = 0; j0 < kend; j0 += kPfKeys) {
+    const float* vl = vt + b * HD + (((DW * part + DT * c) / 4) ^ vsw(b)) * 4 + (DT * c) % 4;  // key b of the tile
+    for (int j0 = 0; j0 < kend; j0 += KT) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();  // the keys are here; the previous values and scores are no longer read
         load_v(j0);
-        float4 sc4 = make_float4(0.f, 0.f, 0.f, 0.f);  // keys 16 hv + 4 b + (0..3) of row c
+        float4 sc4 = make_float4(0.f, 0.f, 0.f, 0.f);  // keys 16 part + 4 b + (0..3) of row c
+        if (j0 + 16 * part < kend) {                    // uniform
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(kt[(16 * hv + c) * HD + 4 * (u ^ c) + b], qv[u], v16f{}, 0, 0, 0);
+            for (int u = 0; u < U; ++u) {
+                const v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(kt[(16 * part + c) * HD + 4 * (u ^ c) + b], qv[u], v16f{}, 0, 0, 0);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                sc4.x += d[4 * k];
-                sc4.y += d[4 * k + 1];
-                sc4.z += d[4 * k + 2];
-                sc4.w += d[4 * k + 3];
+                for (int k = 0; k < 4; ++k) {
+                    sc4.x += d[4 * k];
+                    sc4.y += d[4 * k + 1];
+                    sc4.z += d[4 * k + 2];
+                    sc4.w += d[4 * k + 3];
+                }
             }
         }
-        *(float4*)(st + (16 * rg + c) * kPfSStride + 16 * hv + 4 * b) = sc4;
+        *(float4*)(st + (16 * rg + c) * SS + 16 * part + 4 * b) = sc4;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();  // the scores and values are here; the keys are no longer read
-        if (j0 + kPfKeys < kend) load_k(j0 + kPfKeys);
-        float p[8], bm = -INFINITY;  // key 4 i + b of row c
+        if (j0 + KT < kend) load_k(j0 + KT);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float v = st[(16 * rg + c) * kPfSStride + 4 * i + b];
-            p[i] = j0 + 4 * i + b <= qpos ? v * scale + 0.0f : -INFINITY;
-            bm = fmaxf(bm, p[i]);
-        }
-        float x = bm, y = bm;
-        swap16(x, y);
-        bm = fmaxf(x, y);
-        x = y = bm;
-        swap32(x, y);
-        const float mn = fmaxf(m, fmaxf(x, y));
-        const float corr = mn == -INFINITY ? 1.0f : expf(m - mn);
+        for (int jb = 0; jb < KT; jb += 32) {
+            if (jb > 0 && j0 + jb >= kend) break;  // uniform
+            float p[8], bm = -INFINITY;  // key 4 i + b of row c
 #pragma unroll
-        for (int i = 0; i < 8; ++i) p[i] = p[i] == -INFINITY ? 0.0f : expf(p[i] - mn);
-        // keys 8 b .. 8 b + 7 summed in order by row b of lanes, then the four sums in pairs
-        float ps = 0.0f;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            float a0 = p[h], a1 = p[2 + h], a2 = p[4 + h], a3 = p[6 + h];
-            swap32(a0, a2);
-            swap32(a1, a3);
-            swap16(a0, a1);
-            swap16(a2, a3);
-            ps += a0;
-            ps += a1;
-            ps += a2;
-            ps += a3;
-        }
-        x = y = ps;
-        swap16(x, y);
-        ps = x + y;
-        x = y = ps;
-        swap32(x, y);
-        ps = x + y;
-        l = l * corr + ps;
-        m = mn;
-#pragma unroll
-        for (int t = 0; t < DT; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[t][e] *= corr;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            float vv[DT];
-            const float* vr = vt + (4 * i + b) * HD + (HD / 2) * hv + DT * c;
-            if constexpr (DT == 4) {
-                const float4 f = *(const float4*)vr;
-                vv[0] = f.x, vv[1] = f.y, vv[2] = f.z, vv[3] = f.w;
-            } else {
-                const float2 f = *(const float2*)vr;
-                vv[0] = f.x, vv[1] = f.y;
+            for (int i = 0; i < 8; ++i) {
+                const float v = st[(16 * rg + c) * SS + jb + 4 * i + b];
+                p[i] = j0 + jb + 4 * i + b <= qpos ? v * scale + 0.0f : -INFINITY;
+                bm = fmaxf(bm, p[i]);
             }
+            float x = bm, y = bm;
+            swap16(x, y);
+            bm = fmaxf(x, y);
+            x = y = bm;
+            swap32(x, y);
+            const float mn = fmaxf(m, fmaxf(x, y));
+            const float corr = mn == -INFINITY ? 1.0f : expf(m - mn);
 #pragma unroll
-            for (int t = 0; t < DT; ++t) {
-                const v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(vv[t], p[i], v16f{}, 0, 0, 0);
+            for (int i = 0; i < 8; ++i) p[i] = p[i] == -INFINITY ? 0.0f : expf(p[i] - mn);
+            // keys 8 b .. 8 b + 7 summed in order by row b of lanes, then the four sums in pairs
+            float ps = 0.0f;
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
+            for (int h = 0; h < 2; ++h) {
+                float a0 = p[h], a1 = p[2 + h], a2 = p[4 + h], a3 = p[6 + h];
+                swap32(a0, a2);
+                swap32(a1, a3);
+                swap16(a0, a1);
+                swap16(a2, a3);
+                ps += a0;
+                ps += a1;
+                ps += a2;
+                ps += a3;
+            }
+            x = y = ps;
+            swap16(x, y);
+            ps = x + y;
+            x = y = ps;
+            swap32(x, y);
+            ps = x + y;
+            l = l * corr + ps;
+            m = mn;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) o[t][e] += d[4 * k + e];
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[t][e] *= corr;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                float vv[DT];
+                const float* vr = vl + (jb + 4 * i) * HD;
+                if constexpr (DT == 4) {
+                    const float4 f = *(const float4*)vr;
+                    vv[0] = f.x, vv[1] = f.y, vv[2] = f.z, vv[3] = f.w;
+                } else if constexpr (DT == 2) {
+                    const float2 f = *(const float2*)vr;
+                    vv[0] = f.x, vv[1] = f.y;
+                } else {
+                    vv[0] = *vr;
+                }
+#pragma unroll
+                for (int t = 0; t < DT; ++t) {
+                    const v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(vv[t], p[i], v16f{}, 0, 0, 0);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[t][e] += d[4 * k + e];
+                }
             }
         }
     }
     if (row >= R) return;
-    // o[t][e] is head dim HD / 2 hv + DT (4 b + e) + t: 4 DT consecutive dims a lane
-    float* out = ctx + ((int64_t)(t0 + rr / G) * nh + g * G + rr % G) * HD + (HD / 2) * hv + 4 * DT * b;
+    // o[t][e] is head dim DW part + DT (4 b + e) + t: 4 DT consecutive dims a lane
+    float* out = ctx + ((int64_t)(t0 + rr / G) * nh + g * G + rr % G) * HD + DW * part + 4 * DT * b;
     float f[4 * DT];
 #pragma unroll
     for (int t = 0; t < DT; ++t)
@@ -237,7 +256,8 @@ __global__ __launch_bounds__(256, 3) void k_prefill_attn(const float* __restrict
     for (int i = 0; i < DT; ++i) *(float4*)(out + 4 * i) = make_float4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
 }
 
-// One thread per token t (and per tile index): stream-major order, stream s's tokens at
+// One thread per token t (and per tile index): tiles in descending order of their last position;
+// tokens in stream-major order, stream s's tokens at
 // rows base_s .. base_s + counts[s] - 1 and positions lens[s] .. lens[s] + counts[s] - 1.
 __global__ __launch_bounds__(256) void k_prefill_tables(PrefillMeta pm, int T, int2* __restrict__ tok,
                                                         int4* __restrict__ tiles, int* __restrict__ last) {
@@ -247,8 +267,16 @@ __global__ __launch_bounds__(256) void k_prefill_tables(PrefillMeta pm, int T, i
         const int c = pm.counts[s], nt = (c + pm.tile_tokens - 1) / pm.tile_tokens;
         if (t >= base && t < base + c) tok[t] = make_int2(s, pm.lens[s] + (t - base));
         if (t >= tbase && t < tbase + nt) {
-            const int i0 = (t - tbase) * pm.tile_tokens;
-            tiles[t] = make_int4(s, base + i0, min(pm.tile_tokens, c - i0), pm.lens[s] + i0);
+            const int i0 = (t - tbase) * pm.tile_tokens, cnt = min(pm.tile_tokens, c - i0), kend = pm.lens[s] + i0 + cnt;
+            // its rank: the tiles of every stream that end later, or at the same position in an
+            // earlier stream (a stream's tiles end at lens + tile_tokens, lens + 2 tile_tokens, ...)
+            int rank = 0;
+            for (int z = 0; z < pm.n; ++z) {
+                const int cz = pm.counts[z], nz = (cz + pm.tile_tokens - 1) / pm.tile_tokens;
+                const int d = kend - (z < s ? 1 : 0) - pm.lens[z];  // its tiles that end at or before
+                rank += nz - (d >= cz ? nz : max(d, 0) / pm.tile_tokens);
+            }
+            tiles[rank] = make_int4(s, base + i0, cnt, pm.lens[s] + i0);
         }
         if (t == 0) last[s] = c > 0 ? base + c - 1 : -1;
         base += c;
@@ -307,13 +335,19 @@ hipError_t launch_prefill_attn(const float* q, const float* kc, const float* vc,
     if (!prefill_attn_supported(nh, nkv, hd)) return hipErrorInvalidValue;
     if (n_tiles == 0) return hipSuccess;
     const float scale = (float)(1.0 / sqrt((double)hd));
-    const dim3 grid(n_tiles, nkv, kPfRows / kPfWgRows);
-    if (hd == 128)
-        hipLaunchKernelGGL(k_prefill_attn<128>, grid, dim3(256), 0, s, q, kc, vc, (const int4*)tiles, nh, nkv, max_seq,
-                           kv_stream_stride, scale, ctx);
-    else
-        hipLaunchKernelGGL(k_prefill_attn<64>, grid, dim3(256), 0, s, q, kc, vc, (const int4*)tiles, nh, nkv, max_seq,
-                           kv_stream_stride, scale, ctx);
+    // Head dim 64: four waves per 16 rows while two of them would leave workgroups short of three
+    // per CU (us at 226 tokens of 14 / 2 heads, 104 workgroups by two: 16.4 by four against
+    // 23.5; 700 tokens, 312: 43.6 / 59.6; 1300 in two prompts, 580: 61 / 66; 2400 in two, 1068:
+    // 179 / 165: the softmax is computed by each wave of a row).  At head dim 128 it was never
+    // ahead by more than 5 % (64 KB of tiles leave two workgroups per CU).
+    const bool four = hd == 64 && (int64_t)n_tiles * nkv * 2 <= 768;
+#define SXQ_PF(HD, NP)                                                                                               \
+    hipLaunchKernelGGL((k_prefill_attn<HD, NP>), dim3((unsigned)(n_tiles * nkv * NP)), dim3(256), 0, s, q, kc, vc,   \
+                       (const int4*)tiles, nh, nkv, max_seq, kv_stream_stride, scale, ctx)
+    if (hd == 128) SXQ_PF(128, 2);
+    else if (four) SXQ_PF(64, 4);
+    else SXQ_PF(64, 2);
+#undef SXQ_PF
     return hipGetLastError();
 }
 
