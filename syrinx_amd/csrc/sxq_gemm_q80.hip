@@ -22,8 +22,8 @@
 //    Eight times the parallelism per tile at about twice the work per output: for few tiles.
 // One kernel (64 x 128 tiles, operands one block ahead in registers, 1.1 us per block) for 128
 // rows and more and the GEMV four rows per launch below took: 896 x 4864 at 8 / 50 / 226 rows
-// 12.9 / 69 / 166 us (now 12.1 / 12.8 / 24.4), 9728 x 896 12.5 / 63 / 45 (8.5 / 11.4 / 22.2), 2048 x
-// 1024 Q4_0 at 500 rows 46.7 (14.3), 19456 x 2560 at 16 / 226 rows 92 / 157 (20.9 / 82).
+// 12.9 / 69 / 166 us (now 10.8 / 11.4 / 21.0), 9728 x 896 12.5 / 63 / 45 (7.6 / 10.4 / 20.6), 2048 x
+// 1024 Q4_0 at 500 rows 46.7 (14.7), all with the activation quantizer's launch.
 #include "sxq_kernels.h"
 #include "sxq_quant_dev.h"
 
@@ -35,6 +35,9 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 // Q4_0 nibbles (one per byte, 0..15) as int8 q - 8: (q + 0x78) ^ 0x80 per byte (the add never
 // carries into the next byte).
 SXQ_DEV uint32_t nib_i8(uint32_t q) { return ((q & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u; }
+
+// An f16 block scale as f32, exact: one conversion (f16_bits_to_f32 takes branches).
+SXQ_DEV float f16_scale(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 
 // Workgroups are numbered so that every row tile of one weight tile lands on the same XCD
 // (workgroup id mod 8), whose L2 then serves the weight tile's re-reads.
@@ -53,8 +56,8 @@ constexpr int kSpRow = 20;         // floats per weight row of a block's product
 constexpr int kSpTile = kSpN * kSpRow;
 
 // A chunk is JB consecutive blocks for each wave.  A chunk's weights (1 KB contiguous per
-// Q8_0 row at JB = 4), scales and activation blocks come by coalesced loads, a chunk ahead,
-// into registers and then LDS (rows padded by 16 B: the lanes' operand reads hit every bank
+// Q8_0 row at JB = 4), scales and activation blocks come by coalesced loads, one or two
+// chunks ahead, into registers and then LDS (rows padded by 16 B: the lanes' operand reads hit every bank
 // once).  Loading the operands straight into their lanes instead (16 rows' lines touched per
 // instruction) ran 896 x 4864 at 8 rows in 22.6 us against 12.1.  Lane (r, g) = (lane & 15,
 // lane >> 4) feeds v_mfma_i32_16x16x32_i8 with weight row n0 + r and activation row m0 + r,
@@ -83,7 +86,7 @@ __global__ __launch_bounds__(64 * kSpWaves) void k_gemm_q80_split(const ActQ8_0*
                                                                   const float* __restrict__ bias, const float* res,
                                                                   int64_t ldr) {
     using S = SplitShape<Q4, JB>;
-    constexpr int KC = S::KC, T = S::THREADS;
+    constexpr int KC = S::KC, T = S::THREADS, AHEAD = JB == 4 ? 2 : 1;
     constexpr int NW = (S::WP + T - 1) / T, NA = (S::AP + T - 1) / T, ND = (kSpN * KC + T - 1) / T;
     extern __shared__ __align__(16) char smem[];
     char* sw = smem;                                        // [16][WROW]
@@ -97,44 +100,46 @@ __global__ __launch_bounds__(64 * kSpWaves) void k_gemm_q80_split(const ActQ8_0*
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, g = lane >> 4;
 
-    v4i rw[NW], ra[NA];
-    uint16_t rd[ND];
-    auto stage_load = [&](int c0) {
+    struct Regs {
+        v4i w[NW], a[NA];
+        uint16_t d[ND];
+    };
+    auto stage_load = [&](Regs& k, int c0) {
 #pragma unroll
         for (int i = 0; i < NW; ++i) {  // piece u: row u / (pieces per row), in block order
             constexpr int P = KC * S::WB / 16, PB = S::WB / 16;
             const int u = min(tid + T * i, S::WP - 1), row = u / P, p = u % P;
             const int64_t b = (int64_t)min(n0 + row, N - 1) * nb + min(c0 + p / PB, nb - 1);
-            rw[i] = *(const v4i*)(wqs + b * S::WB + 16 * (p % PB));
+            k.w[i] = *(const v4i*)(wqs + b * S::WB + 16 * (p % PB));
         }
 #pragma unroll
         for (int i = 0; i < ND; ++i) {
             const int u = min(tid + T * i, kSpN * KC - 1);
-            rd[i] = wd[(int64_t)min(n0 + u / KC, N - 1) * nb + min(c0 + u % KC, nb - 1)];
+            k.d[i] = wd[(int64_t)min(n0 + u / KC, N - 1) * nb + min(c0 + u % KC, nb - 1)];
         }
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int u = min(tid + T * i, S::AP - 1), row = u / (3 * KC), p = u % (3 * KC);
             const ActQ8_0* ab = act + (int64_t)min(m0 + row, M - 1) * nb + min(c0 + p / 3, nb - 1);
-            ra[i] = *((const v4i*)ab + p % 3);
+            k.a[i] = *((const v4i*)ab + p % 3);
         }
     };
-    auto stage_store = [&]() {
+    auto stage_store = [&](const Regs& k) {
 #pragma unroll
         for (int i = 0; i < NW; ++i) {
             constexpr int P = KC * S::WB / 16;
             const int u = min(tid + T * i, S::WP - 1);
-            *(v4i*)(sw + (u / P) * S::WROW + 16 * (u % P)) = rw[i];
+            *(v4i*)(sw + (u / P) * S::WROW + 16 * (u % P)) = k.w[i];
         }
 #pragma unroll
         for (int i = 0; i < ND; ++i) {
             const int u = min(tid + T * i, kSpN * KC - 1);
-            sd[(u / KC) * (KC + 1) + u % KC] = f16_bits_to_f32(rd[i]);
+            sd[(u / KC) * (KC + 1) + u % KC] = f16_scale(k.d[i]);
         }
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int u = min(tid + T * i, S::AP - 1);
-            *(v4i*)(sa + (u / (3 * KC)) * S::AROW + 16 * (u % (3 * KC))) = ra[i];
+            *(v4i*)(sa + (u / (3 * KC)) * S::AROW + 16 * (u % (3 * KC))) = k.a[i];
         }
     };
     auto products = [&]() {
@@ -179,11 +184,10 @@ __global__ __launch_bounds__(64 * kSpWaves) void k_gemm_q80_split(const ActQ8_0*
     const float* pc = pr + on * kSpRow + om;
     const bool fold = tid < 256;
     float acc = 0.0f;
-    stage_load(0);
-    for (int c0 = 0; c0 < nb; c0 += KC) {
-        stage_store();  // the previous chunk's operand reads are behind its second barrier
+    auto chunk = [&](Regs& k, int c0) {
+        stage_store(k);  // the previous chunk's operand reads are behind its second barrier
         lds_barrier();
-        stage_load(c0 + KC);
+        if (c0 + AHEAD * KC < nb) stage_load(k, c0 + AHEAD * KC);  // uniform
         products();
         lds_barrier();
         if (fold) {
@@ -196,6 +200,22 @@ __global__ __launch_bounds__(64 * kSpWaves) void k_gemm_q80_split(const ActQ8_0*
                 for (int b = 0; b < kc; ++b) acc = acc + pc[b * kSpTile];
             }
         }
+    };
+    // Where a workgroup has its CU to itself (JB = 4) the loads go two chunks ahead: a chunk takes
+    // less time than they do (896 x 4864 at 8 rows 11.5 -> 10.9 us).  With three workgroups per
+    // CU the others cover them (2560 x 9728 at 32 rows 26.9 us, 29.0 with two sets of registers).
+    Regs k0;
+    stage_load(k0, 0);
+    if constexpr (AHEAD == 2) {
+        Regs k1;
+        if (KC < nb) stage_load(k1, KC);
+        for (int c0 = 0; c0 < nb; c0 += 2 * KC) {
+            chunk(k0, c0);
+            if (c0 + KC >= nb) break;  // uniform
+            chunk(k1, c0 + KC);
+        }
+    } else {
+        for (int c0 = 0; c0 < nb; c0 += KC) chunk(k0, c0);
     }
     const int m = m0 + om, n = n0 + on;
     if (fold && m < M && n < N) {
@@ -264,7 +284,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80(const ActQ8_0* __restrict__
 #pragma unroll
         for (int i = 0; i < 2; ++i) *(v4i*)(sa[st] + slot(pr + 32 * i, p)) = ra[i];
         sda[st][jb][jr] = rda;
-        sdw[st][jb][jr] = f16_bits_to_f32(rdw);
+        sdw[st][jb][jr] = f16_scale(rdw);
         if (Q4) {  // element j is the low nibble of byte j, j + 16 the high one
             v4i lo, hi;
 #pragma unroll
@@ -398,7 +418,20 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
     // staging roles: pieces p and p + 8 (blocks p / 2 and p / 2 + 4) of row pr; block jb of row
     // jr (scales, Q4_0 blocks).  Clamped rows and blocks (never used or stored).
     const int pr = tid >> 3, p = tid & 7, jr = tid >> 3, jb = tid & 7;
-    const int64_t arow = (int64_t)min(m0 + pr, M - 1) * nb, brow = (int64_t)min(n0 + pr, N - 1) * nb;
+    // A thread's offsets into the tile's rows stay; a stage only moves the scalar offset.  What
+    // lies past the tile's rows loads as zero, what lies past a row is the next one's: neither
+    // is added or stored.
+    const int rm = min(kMdT, M - m0), rn = min(kMdT, N - n0);
+    constexpr uint32_t AB = sizeof(ActQ8_0), WB = Q4 ? 16 : 32;
+    auto rsrc = [](const void* p, uint32_t bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t ars = rsrc(act + (int64_t)m0 * nb, (uint32_t)(rm * nb) * AB);
+    const __amdgpu_buffer_rsrc_t wrs = rsrc(wqs + (int64_t)n0 * nb * WB, (uint32_t)(rn * nb) * WB);
+    const __amdgpu_buffer_rsrc_t drs = rsrc(wd + (int64_t)n0 * nb, (uint32_t)(rn * nb) * 2u);
+    const uint32_t oa = (uint32_t)(pr * nb + (p >> 1)) * AB + 16u * (p & 1), oda = (uint32_t)(jr * nb + jb) * AB + 32u;
+    const uint32_t ow = Q4 ? (uint32_t)(jr * nb + jb) * 16u : (uint32_t)(pr * nb + (p >> 1)) * 32u + 16u * (p & 1);
+    const uint32_t odw = (uint32_t)(jr * nb + jb) * 2u;
     struct Regs {
         v4i a[2], b[2];
         float da;
@@ -407,14 +440,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
     auto load = [&](Regs& k, int c0) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int b = min(c0 + 4 * i + (p >> 1), nb - 1);
-            k.a[i] = *(const v4i*)(act[arow + b].qs + 16 * (p & 1));
-            if (!Q4) k.b[i] = *(const v4i*)(wqs + (brow + b) * 32 + 16 * (p & 1));
+            k.a[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ars, oa + 4 * i * AB, c0 * AB, 0));
+            if (!Q4) k.b[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, ow + 128u * i, c0 * WB, 0));
         }
-        const int b = min(c0 + jb, nb - 1);
-        k.da = act[arow + b].d;
-        k.dw = wd[brow + b];
-        if (Q4) k.b[0] = *(const v4i*)(wqs + (brow + b) * 16);
+        k.da = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ars, oda, c0 * AB, 0));
+        k.dw = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(drs, odw, c0 * 2, 0);
+        if (Q4) k.b[0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, ow, c0 * WB, 0));
     };
     auto slot = [](int row, int piece) { return row * 256 + ((piece ^ (row & 15)) << 4); };
     auto store = [&](const Regs& k, int st) {
@@ -424,7 +455,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
             if (!Q4) *(v4i*)(sb[st] + slot(pr, p + 8 * i)) = k.b[i];
         }
         sda[st][jb][jr] = k.da;
-        sdw[st][jb][jr] = f16_bits_to_f32(k.dw);
+        sdw[st][jb][jr] = f16_scale(k.dw);
         if (Q4) {  // element j is the low nibble of byte j, j + 16 the high one
             v4i lo, hi;
 #pragma unroll
@@ -438,24 +469,53 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
     };
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     const v4i zero = {};
-    auto block = [&](int st, int j) {  // lane (r, g): elements 8g .. 8g + 7 of both rows
-        const long a = *(const long*)(sa[st] + slot(wm + r, 2 * j + (g >> 1)) + 8 * (g & 1));
-        const long b = *(const long*)(sb[st] + slot(wn + r, 2 * j + (g >> 1)) + 8 * (g & 1));
-        const float4 da = *(const float4*)&sda[st][j][wm + 4 * g];
-        const float dw = sdw[st][j][wn + r];
-        const v4i s = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, zero, 0, 0, 0);
-        acc[0] = acc[0] + ((float)s[0] * dw) * da.x;
-        acc[1] = acc[1] + ((float)s[1] * dw) * da.y;
-        acc[2] = acc[2] + ((float)s[2] * dw) * da.z;
-        acc[3] = acc[3] + ((float)s[3] * dw) * da.w;
+    struct Block {
+        long a, b;
+        float4 da;
+        float dw;
     };
+    auto read = [&](Block& k, int st, int j) {  // lane (r, g): elements 8g .. 8g + 7 of both rows
+        k.a = *(const long*)(sa[st] + slot(wm + r, 2 * j + (g >> 1)) + 8 * (g & 1));
+        k.b = *(const long*)(sb[st] + slot(wn + r, 2 * j + (g >> 1)) + 8 * (g & 1));
+        k.da = *(const float4*)&sda[st][j][wm + 4 * g];
+        k.dw = sdw[st][j][wn + r];
+    };
+    auto dots = [&](const Block& k) { return __builtin_amdgcn_mfma_i32_16x16x32_i8(k.a, k.b, zero, 0, 0, 0); };
+    auto fold = [&](const Block& k, const v4i& s) {
+        acc[0] = acc[0] + ((float)s[0] * k.dw) * k.da.x;
+        acc[1] = acc[1] + ((float)s[1] * k.dw) * k.da.y;
+        acc[2] = acc[2] + ((float)s[2] * k.dw) * k.da.z;
+        acc[3] = acc[3] + ((float)s[3] * k.dw) * k.da.w;
+    };
+    // Four blocks' operands are read and multiplied together, and the next four read while
+    // they are folded: a wave often has its SIMD to itself, and block by block it waited for
+    // LDS and the matrix cores at each (896 x 4864 at 226 rows 24.9 us, now 21.0).
     auto compute = [&](int st, int c) {
         const int kc = nb - c * kMdKC;
         if (kc >= kMdKC) {
+            Block k[4], n[4];
+            v4i s[4];
 #pragma unroll
-            for (int j = 0; j < kMdKC; ++j) block(st, j);
+            for (int j = 0; j < 4; ++j) read(k[j], st, j);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] = dots(k[j]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) read(n[j], st, 4 + j);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) fold(k[j], s[j]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] = dots(n[j]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) fold(n[j], s[j]);
         } else {
-            for (int j = 0; j < kc; ++j) block(st, j);
+            for (int j = 0; j < kc; ++j) {
+                Block k;
+                read(k, st, j);
+                fold(k, dots(k));
+            }
         }
     };
 
@@ -508,7 +568,8 @@ static hipError_t gemm_q80_dispatch(const QWeight& w, const ActQ8_0* act, int m,
         return hipGetLastError();                                                                            \
     } while (0)
     // The kernel by the number of 16 x 16 tiles, T, and of 64 x 64 tiles (us with the
-    // activation quantizer's launch, in a graph; split by blocks / mid / 64 x 64):
+    // activation quantizer's launch, in a graph; split by blocks / mid / 64 x 64, before each of
+    // them became 3 to 15 % faster):
     //  T <= 256, a workgroup per CU: the split kernel with 32-block chunks (896 x 4864 at 64
     //  rows, T = 224: 12.9 / 22.6 / 48; 2048 x 1024 Q4_0 at 32 rows, T = 256: 6.4 / 9.1 / 16);
     //  T <= 768: with 16-block chunks, three workgroups per CU (9728 x 896 at 16 rows, T = 608:

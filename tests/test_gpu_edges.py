@@ -101,7 +101,7 @@ def test_bf16_rows_quantized_directly(cuda, dt, k, m):
         assert torch.equal(qmm.forward(x), qmm.forward(x.float()))
 
 
-@pytest.mark.parametrize("hd,G,nkv", [(128, 4, 2), (64, 7, 2), (128, 1, 2), (64, 64, 1), (128, 5, 1)])
+@pytest.mark.parametrize("hd,G,nkv", [(128, 4, 2), (64, 7, 2), (128, 1, 2), (64, 64, 1), (128, 5, 1), (64, 64, 2)])
 def test_prefill_attention_tiles(cuda, hd, G, nkv):
     """Causal attention of ragged prompts on top of filled caches against 64 bits: prompts of one
     token, of a partial and of several row tiles, caches that end inside a key tile."""
