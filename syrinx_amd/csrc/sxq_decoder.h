@@ -85,11 +85,12 @@ hipError_t launch_prefill_rope_kv(const float* qkv, int T, int qkv_n, int nh, in
                                   const int* tok, float* qout, float* kc, float* vc, int64_t kv_stream_stride,
                                   int max_seq, hipStream_t s);
 // Causal GQA attention of the prompt's queries over each stream's cache; tiles[4 i ..]
-// = {stream, first token row, token count (<= prefill_tile_tokens), first position}.
+// = {stream, first token row, token count (<= prefill_tile_tokens), first position}.  The
+// context goes to ctx (f32 rows) and, as Q8_0 activation blocks, to act; either may be null.
 bool prefill_attn_supported(int nh, int nkv, int hd);
 int prefill_tile_tokens(int nh, int nkv);
 hipError_t launch_prefill_attn(const float* q, const float* kc, const float* vc, const int* tiles, int n_tiles, int nh,
-                               int nkv, int hd, int max_seq, int64_t kv_stream_stride, float* ctx, hipStream_t s);
+                               int nkv, int hd, int max_seq, int64_t kv_stream_stride, float* ctx, void* act, hipStream_t s);
 // The token and tile tables of one prefill, built on the device from the per-stream
 // token counts and cache lengths (streams 0 .. n-1, tokens stream-major): tok (2 ints per
 // token), tiles (4 ints per tile, at most T + n tiles), last[s] = row of stream s's last

@@ -528,6 +528,9 @@ hipError_t enqueue_prefill(sxq_lm* lm, const PrefillMeta& pm, int T, const int* 
     // the SiLU * mul quantizer, three conversions of f32 rows and the context's quantizer:
     // four layers 3653 -> 3244 us.
     const bool f16 = c.weight_dtype == kQ4K && !exact && T >= kGemmMinRows && c.dim <= kPrepMaxK && I <= kPrepMaxK;
+    // otherwise the f32 rows are read by a trace, or by the f16 product of rows over kPrepMaxK
+    const bool f32_rows = tr || (c.weight_dtype == kQ4K && !exact && T >= kGemmMinRows);
+    const bool ctx_blocks = lm->vdt == kQ8_0;  // the attention leaves the context quantized
     // y = rmsnorm(h) . W^T (+ bias); hn keeps the f32 rows where `keep` or a trace reads them
     auto norm_proj = [&](const QWeight& w, const float* nw, float* y, const float* bias, bool keep) -> hipError_t {
         hipError_t r;
@@ -541,7 +544,7 @@ hipError_t enqueue_prefill(sxq_lm* lm, const PrefillMeta& pm, int T, const int* 
             if (r == hipSuccess) r = launch_gemm_q4k(w, gws, T, y, w.n, bias, nullptr, w.n, s);
             return r;
         }
-        r = launch_rmsnorm_quant(lm->vdt, h, T, c.dim, nw, c.norm_eps, act, hn, s);
+        r = launch_rmsnorm_quant(lm->vdt, h, T, c.dim, nw, c.norm_eps, act, keep || f32_rows ? hn : nullptr, s);
         return r == hipSuccess ? pf_proj(lm, w, hn, act, T, y, bias, nullptr, exact, gws, s) : r;
     };
     for (int l = 0; l < c.n_layers; ++l) {
@@ -557,9 +560,9 @@ hipError_t enqueue_prefill(sxq_lm* lm, const PrefillMeta& pm, int T, const int* 
                                   lm->kv_stream_stride, c.max_seq, s));
         PF(record(q, (size_t)T * lm->ctx));
         PF(launch_prefill_attn(q, kc, vc, tiles, n_tiles, c.n_heads, c.n_kv_heads, c.head_dim, c.max_seq,
-                               lm->kv_stream_stride, cx, s));
+                               lm->kv_stream_stride, ctx_blocks && !tr ? nullptr : cx, ctx_blocks ? act : nullptr, s));
         PF(record(cx, (size_t)T * lm->ctx));
-        if (!f16) PF(launch_quantize_act(lm->vdt, false, cx, lm->ctx, T, lm->ctx, act, s));
+        if (!f16 && !ctx_blocks) PF(launch_quantize_act(lm->vdt, false, cx, lm->ctx, T, lm->ctx, act, s));
         PF(pf_proj(lm, L.wo.w, cx, act, T, h, L.bo, h, exact, gws, s));
         PF(record(h, Td));
         PF(norm_proj(L.w13.w, L.ffn_norm, gu, nullptr, false));
@@ -569,7 +572,7 @@ hipError_t enqueue_prefill(sxq_lm* lm, const PrefillMeta& pm, int T, const int* 
             PF(launch_gemm_q4k_prep_silu(gu, T, L.w2.w.n, I, gws, tr ? af : nullptr, s));
             PF(launch_gemm_q4k(L.w2.w, gws, T, h, c.dim, nullptr, h, c.dim, s));
         } else {
-            PF(launch_silu_mul_quant(lm->vdt, gu, T, I, act, af, s));
+            PF(launch_silu_mul_quant(lm->vdt, gu, T, I, act, f32_rows ? af : nullptr, s));
             PF(pf_proj(lm, L.w2.w, af, act, T, h, nullptr, h, exact, gws, s));
         }
         PF(record(af, (size_t)T * I));

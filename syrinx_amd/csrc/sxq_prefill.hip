@@ -96,7 +96,8 @@ template <int HD, int NP>
 __global__ __launch_bounds__(256, 3) void k_prefill_attn(const float* __restrict__ q, const float* __restrict__ kc,
                                                          const float* __restrict__ vc, const int4* __restrict__ tiles,
                                                          int nh, int nkv, int max_seq, int64_t kv_stream_stride,
-                                                         float scale, float* __restrict__ ctx) {
+                                                         float scale, float* __restrict__ ctx,
+                                                         ActQ8_0* __restrict__ act) {
     constexpr int KT = 16 * NP, RW = 64 / NP;     // keys and rows per workgroup
     constexpr int U = HD / 4, DW = HD / NP, DT = DW / 16;  // head-dim quads; dims of a wave's outputs, in 16s
     constexpr int SS = KT + 4;  // floats per row of scores: float4-aligned, the reads hit 64 banks
@@ -244,16 +245,32 @@ __global__ __launch_bounds__(256, 3) void k_prefill_attn(const float* __restrict
             }
         }
     }
-    if (row >= R) return;
     // o[t][e] is head dim DW part + DT (4 b + e) + t: 4 DT consecutive dims a lane
-    float* out = ctx + ((int64_t)(t0 + rr / G) * nh + g * G + rr % G) * HD + DW * part + 4 * DT * b;
+    const int d0 = DW * part + 4 * DT * b;
     float f[4 * DT];
 #pragma unroll
     for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) f[DT * e + t] = o[t][e] / l;
+    auto head_row = [&](int r) { return (int64_t)(t0 + r / G) * nh + g * G + r % G; };  // of the context
+    if (ctx && row < R) {
+        float* out = ctx + head_row(rr) * HD + d0;
 #pragma unroll
-    for (int i = 0; i < DT; ++i) *(float4*)(out + 4 * i) = make_float4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
+        for (int i = 0; i < DT; ++i) *(float4*)(out + 4 * i) = make_float4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
+    }
+    if (!act) return;  // uniform
+    // the context's Q8_0 blocks for the O projection: the rows meet in kt (read last before the
+    // loop's last barrier), 256 elements of them to a wave at a time
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+        *(float4*)(kt + (16 * rg + c) * HD + d0 + 4 * i) = make_float4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < RW * HD / 1024; ++i) {
+        const int e = 256 * (wave + 4 * i) + 4 * lane, r = r0 + e / HD;
+        ActQ8_0* block = act + head_row(min(r, R - 1)) * (HD / 32) + (e % HD) / 32;
+        wave_quantize_q8_0_block<false>(*(const float4*)(kt + e), lane, r < R, block);
+    }
 }
 
 // One thread per token t (and per tile index): tiles in descending order of their last position;
@@ -331,7 +348,7 @@ bool prefill_attn_supported(int nh, int nkv, int hd) { return (hd == 64 || hd ==
 int prefill_tile_tokens(int nh, int nkv) { return kPfRows / (nh / nkv); }
 
 hipError_t launch_prefill_attn(const float* q, const float* kc, const float* vc, const int* tiles, int n_tiles, int nh,
-                               int nkv, int hd, int max_seq, int64_t kv_stream_stride, float* ctx, hipStream_t s) {
+                               int nkv, int hd, int max_seq, int64_t kv_stream_stride, float* ctx, void* act, hipStream_t s) {
     if (!prefill_attn_supported(nh, nkv, hd)) return hipErrorInvalidValue;
     if (n_tiles == 0) return hipSuccess;
     const float scale = (float)(1.0 / sqrt((double)hd));
@@ -343,7 +360,7 @@ hipError_t launch_prefill_attn(const float* q, const float* kc, const float* vc,
     const bool four = hd == 64 && (int64_t)n_tiles * nkv * 2 <= 768;
 #define SXQ_PF(HD, NP)                                                                                               \
     hipLaunchKernelGGL((k_prefill_attn<HD, NP>), dim3((unsigned)(n_tiles * nkv * NP)), dim3(256), 0, s, q, kc, vc,   \
-                       (const int4*)tiles, nh, nkv, max_seq, kv_stream_stride, scale, ctx)
+                       (const int4*)tiles, nh, nkv, max_seq, kv_stream_stride, scale, ctx, (ActQ8_0*)act)
     if (hd == 128) SXQ_PF(128, 2);
     else if (four) SXQ_PF(64, 4);
     else SXQ_PF(64, 2);

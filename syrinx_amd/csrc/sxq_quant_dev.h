@@ -209,10 +209,11 @@ SXQ_DEV void wave_quantize_q8k(float4 v, int lane, void* out, MmaRec* rec = null
     wave_quantize_q8k_n<1, CANON>(vv, lane, oo, ok, rr, rec_row);
 }
 
-// Quantize 256 consecutive activations (8 Q8_0 blocks; lanes 8b..8b+7 own block b) to
-// Q8_0: k_quants.rs BlockQ8_0::from_float.  `valid` = this lane's block lies inside k.
+// Quantize eight blocks of 32 activations (lanes 8b..8b+7 own block b, four elements each, and
+// write it to `block`) to Q8_0: k_quants.rs BlockQ8_0::from_float.  `valid` = this lane's block
+// is to be written.
 template <bool CANON>
-SXQ_DEV void wave_quantize_q8_0(float4 v, int lane, bool valid, void* out) {
+SXQ_DEV void wave_quantize_q8_0_block(float4 v, int lane, bool valid, void* block) {
     const float x[4] = {v.x, v.y, v.z, v.w};
     float am = 0.0f;
 #pragma unroll
@@ -231,24 +232,31 @@ SXQ_DEV void wave_quantize_q8_0(float4 v, int lane, bool valid, void* out) {
     s += dpp_i32<0x4E>(s);
     s += dpp_i32<0x141>(s);
     if (!valid) return;
-    const int blk = lane >> 3, w = lane & 7;
+    const int w = lane & 7;
     const uint32_t packed = (uint32_t)(q[0] & 0xFF) | ((uint32_t)(q[1] & 0xFF) << 8) |
                             ((uint32_t)(q[2] & 0xFF) << 16) | ((uint32_t)(q[3] & 0xFF) << 24);
     if (CANON) {
         // 34-byte blocks are only 2-byte aligned: write halves.
-        BlockQ8_0* b = (BlockQ8_0*)out + blk;
+        BlockQ8_0* b = (BlockQ8_0*)block;
         uint16_t* qs16 = (uint16_t*)b->qs;
         qs16[2 * w] = (uint16_t)(packed & 0xFFFF);
         qs16[2 * w + 1] = (uint16_t)(packed >> 16);
         if (w == 0) b->d = dh;
     } else {
-        ActQ8_0* b = (ActQ8_0*)out + blk;
+        ActQ8_0* b = (ActQ8_0*)block;
         ((uint32_t*)b->qs)[w] = packed;
         if (w == 0) {
             b->d = f16_bits_to_f32(dh);
             b->asum = s;
         }
     }
+}
+
+// 256 consecutive activations: eight consecutive blocks at `out`.
+template <bool CANON>
+SXQ_DEV void wave_quantize_q8_0(float4 v, int lane, bool valid, void* out) {
+    const int blk = lane >> 3;
+    wave_quantize_q8_0_block<CANON>(v, lane, valid, CANON ? (void*)((BlockQ8_0*)out + blk) : (void*)((ActQ8_0*)out + blk));
 }
 
 }  // namespace sxq

@@ -114,7 +114,10 @@ def test_prefill_attention_tiles(cuda, hd, G, nkv):
     for counts in ([1, 31, 64, 130], [70, 33, 1, 65]):  # the second call starts at the first's lengths
         pos0 = lm.lengths(4)
         xs = [torch.randn(c, cfg.dim, generator=gen, device=cuda) * 3 for c in counts]
-        tr = lm.prefill(embeds=xs, all_logits=True, trace=True)[3]["layers"][0]
+        logits, _, _, tr = lm.prefill(embeds=xs, all_logits=True, trace=True)
+        tr = tr["layers"][0]
+        if pos0[0] == 0:
+            first = xs, logits
         q = torch.from_numpy(tr["q"]).to(cuda).double().view(-1, G * nkv, hd)
         got = torch.from_numpy(tr["ctx"]).to(cuda).double().view(-1, G * nkv, hd)
         at = 0
@@ -131,6 +134,8 @@ def test_prefill_attention_tiles(cuda, hd, G, nkv):
                     err = (got[at:at + c, g * G + h] - want).abs().max()
                     assert err <= tol, f"counts {counts} stream {s} head {g * G + h}: {float(err):.3g} > {float(tol):.3g}"
             at += c
+    lm.reset(4)  # without a trace the context goes to the O projection as blocks only
+    assert torch.equal(lm.prefill(embeds=first[0], all_logits=True)[0], first[1])
 
 
 @pytest.mark.parametrize("dt,k", [(G.Q4K, 512), (G.Q8_0, 896), (G.Q4_0, 320)])
