@@ -176,11 +176,16 @@ SXQ_DEV int nearest_int(float v) {
     const float r = roundf(v);
     return r != r ? 0 : (r >= 2147483647.0f ? 2147483647 : (r <= -2147483648.0f ? (int)0x80000000u : (int)r));
 }
-// nearest_int(v) clamped to 0..15, as a float: half-away rounding only matters above zero
-// (v - trunc(v) is exact), a NaN gives 0 and an infinity its bound, as the clamped int does.
-SXQ_DEV float level15(float v) {
-    const float t = truncf(v);
-    return fminf(fmaxf(t + (v - t >= 0.5f ? 1.0f : 0.0f), 0.0f), 15.0f);
+// nearest_int(v) clamped to 0..15, as a float: half-away rounding only matters above zero, where
+// it is trunc(v + the float below 0.5) (checked for every f32); a NaN gives 0 and an infinity
+// its bound, as the clamped int does.
+SXQ_DEV float level15(float v) { return __builtin_amdgcn_fmed3f(truncf(v + 0x1.fffffep-2f), 0.0f, 15.0f); }
+// level15(a / d), y = RN(1 / d): with a faithful q0 = a y the quotient rounded once is
+// q0 + (a - q0 d) y (Markstein); a q0 too large for that (or not finite) is at a bound anyway.
+SXQ_DEV float level15_div(float a, float d, float y) {
+    const float q0 = a * y;
+    const float q = __builtin_fmaf(__builtin_fmaf(-d, q0, a), y, q0);
+    return level15(fabsf(q0) < 32.0f ? q : q0);
 }
 // f32 bits <-> the integer of the same total order (its own inverse)
 SXQ_DEV int total_key(int a) { return a ^ (int)(((unsigned)(a >> 31)) >> 1); }
@@ -203,7 +208,7 @@ SXQ_DEV void make_qkx1_quants(const float (&x)[32], float* scale_out, float* min
     float iscale = 15.0f / (mx - min);
     float scale = 0.0f;
     for (int it = 0; it < 5; ++it) {
-        float sumlx = 0.0f, suml2 = 0.0f;  // suml2: at most 32 * 225, exact
+        float sumlx = 0.0f, suml2 = 0.0f;  // suml2: at most 32 * 225, exact either way
         bool changed = false;
 #pragma unroll
         for (int i = 0; i < 32; ++i) {
@@ -212,7 +217,7 @@ SXQ_DEV void make_qkx1_quants(const float (&x)[32], float* scale_out, float* min
             changed = changed || li != L[i];
             L[i] = li;
             sumlx += dx * li;
-            suml2 += li * li;
+            suml2 = __builtin_fmaf(li, li, suml2);
         }
         scale = sumlx / suml2;
         float sum = -0.0f;
@@ -242,7 +247,9 @@ SXQ_DEV void get_scale_min_k4(int j, const uint8_t* q, int& d, int& m) {
 // nibbles.  The search is a serial chain of float sums per sub-block (up to 5 x 64 adds in
 // Candle's order), so the parallelism is over sub-blocks: VALU-bound.  With a workgroup per
 // super-block (eight of its 256 threads searching) a 2560 x 9728 matrix took 9666 us;
-// this runs it in 56-64 us.  V: x and out are 16-byte aligned; otherwise element loads and
+// this runs it in 49 us
+// (56 with the rounding and the final divisions spelled out: 16 VALU operations per element and
+// round where there are 12 now).  V: x and out are 16-byte aligned; otherwise element loads and
 // byte stores.
 template <bool V>
 __global__ __launch_bounds__(256) void k_from_float_q4k(const float* __restrict__ x, int64_t nblocks,
@@ -282,13 +289,14 @@ __global__ __launch_bounds__(256) void k_from_float_q4k(const float* __restrict_
     const uint16_t dh = f32_to_f16_bits(max_scale / 63.0f), mh = f32_to_f16_bits(max_min / 63.0f);
     const float d = f16_bits_to_f32(dh) * (float)sc;
     const float dm = f16_bits_to_f32(mh) * (float)m;
+    const float y = 1.0f / d;
     uint32_t w[8];  // this sub-block's levels, a byte each
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         w[i] = 0;
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-            if (d != 0.0f) w[i] |= (uint32_t)level15((xs[4 * i + t] + dm) / d) << (8 * t);
+            if (d != 0.0f) w[i] |= (uint32_t)level15_div(xs[4 * i + t] + dm, d, y) << (8 * t);
     }
     // byte l of 64-element chunk c: sub-block 2c's level l below, 2c + 1's above; the lower
     // lane of a pair stores the first 16 bytes of the chunk, the upper one the rest
