@@ -416,7 +416,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
     const int r = lane & 15, g = lane >> 4;
 
     // staging roles: pieces p and p + 8 (blocks p / 2 and p / 2 + 4) of row pr; block jb of row
-    // jr (scales, Q4_0 blocks).  Clamped rows and blocks (never used or stored).
+    // jr (scales, Q4_0 blocks)
     const int pr = tid >> 3, p = tid & 7, jr = tid >> 3, jb = tid & 7;
     // A thread's offsets into the tile's rows stay; a stage only moves the scalar offset.  What
     // lies past the tile's rows loads as zero, what lies past a row is the next one's: neither

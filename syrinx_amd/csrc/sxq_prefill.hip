@@ -72,6 +72,18 @@ SXQ_DEV void pf_tile_to_lds(__amdgpu_buffer_rsrc_t src, float* dst, int wave, in
     }
 }
 
+// Zeroes rows `from` and up among the pieces this wave loaded (whose loads have completed), so
+// that a probability of zero never meets an infinite value.
+template <int HD, int ROWS>
+SXQ_DEV void pf_zero_rows(float* dst, int wave, int lane, int from) {
+    constexpr int PR = HD / 4, NI = ROWS * PR / 256;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int at = (wave * NI + i) * 64 + lane;
+        if (at / PR >= from) *(float4*)(dst + 4 * at) = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+}
+
 // One workgroup (256 threads) per (tile, KV group, share of the tile's rows): a tile is up to
 // kPfRows / G consecutive prompt tokens of one stream (tile = {stream, first token row t0,
 // count, position p0 of token t0}); its rows are r = i * G + hh (token i, query head
@@ -133,7 +145,7 @@ __global__ __launch_bounds__(256, 3) void k_prefill_attn(const float* __restrict
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kc + koff), (short)0, (int)((uint32_t)kend * HD * 4u), 0x00020000);
     const __amdgpu_buffer_rsrc_t vrs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vc + koff), (short)0, (int)((uint32_t)kend * HD * 4u), 0x00020000);
-    // keys past the last one load it again (their probabilities are zero)
+    // keys past the last one load it again (their scores are masked, their values zeroed)
     auto load_k = [&](int j0) {
         pf_tile_to_lds<HD, KT>(krs, kt, wave, lane, [&](int r) { return (uint32_t)min(j0 + r, kend - 1) * (HD * 4u); }, ksw);
     };
@@ -174,6 +186,7 @@ __global__ __launch_bounds__(256, 3) void k_prefill_attn(const float* __restrict
         }
         *(float4*)(st + (16 * rg + c) * SS + 16 * part + 4 * b) = sc4;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (j0 + KT > kend) pf_zero_rows<HD, KT>(vt, wave, lane, kend - j0);  // uniform: the last tile
         lds_barrier();  // the scores and values are here; the keys are no longer read
         if (j0 + KT < kend) load_k(j0 + KT);
 #pragma unroll

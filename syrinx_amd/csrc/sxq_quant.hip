@@ -246,11 +246,10 @@ SXQ_DEV void get_scale_min_k4(int j, const uint8_t* q, int& d, int& m) {
 // of a super-block share the scale search's results by shuffles and each packs its own
 // nibbles.  The search is a serial chain of float sums per sub-block (up to 5 x 64 adds in
 // Candle's order), so the parallelism is over sub-blocks: VALU-bound.  With a workgroup per
-// super-block (eight of its 256 threads searching) a 2560 x 9728 matrix took 9666 us;
-// this runs it in 49 us
-// (56 with the rounding and the final divisions spelled out: 16 VALU operations per element and
-// round where there are 12 now).  V: x and out are 16-byte aligned; otherwise element loads and
-// byte stores.
+// super-block (eight of its 256 threads searching) a 2560 x 9728 matrix took 9666 us; this runs
+// it in 49 us (56 with the rounding and the final divisions spelled out: 16 VALU operations per
+// element and round where there are 12 now).  V: x and out are 16-byte aligned; otherwise
+// element loads and byte stores.
 template <bool V>
 __global__ __launch_bounds__(256) void k_from_float_q4k(const float* __restrict__ x, int64_t nblocks,
                                                         uint8_t* __restrict__ out) {

@@ -23,7 +23,7 @@ from typing import Sequence
 
 import torch
 
-from ._lib import BF16_INPUT, BIT_EXACT, HOST_PTRS, SxqError, check, lib
+from ._lib import BF16_INPUT, BIT_EXACT, ERR_OOM, HOST_PTRS, SxqError, check, lib
 
 
 class GgmlDType(enum.IntEnum):
@@ -264,7 +264,10 @@ class QMatMul:
         # capture it comes from the graph's memory pool and lives as long as the captured
         # output y (as a graph's own intermediates do), so a caller that re-captures and drops
         # the old outputs releases the old workspaces with them.
-        ws = torch.empty(max(need.value, 1), dtype=torch.uint8, device=xs.device)
+        try:
+            ws = torch.empty(max(need.value, 1), dtype=torch.uint8, device=xs.device)
+        except torch.OutOfMemoryError as e:
+            raise SxqError(ERR_OOM, f"qmm_forward: workspace: {e}") from None
         check(lib().sxq_qmm_forward_ws(self._h, _ptr(xs), shape, dims, strides, _ptr(y), bptr, flags, _ptr(ws),
                                        ws.numel(), _stream_ptr(xs.device)))
         if capturing:
