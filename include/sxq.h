@@ -125,7 +125,9 @@ sxq_status sxq_qmm_forward(const sxq_qmm *qmm, const float *x, const int64_t *x_
                            const int64_t *x_strides, float *y, const float *bias, unsigned flags, void *stream);
 
 /* Device workspace bytes sxq_qmm_forward_ws needs for m rows of x (with `flags` as the
- * forward will get them).  No reference counterpart: Candle allocates inside forward. */
+ * forward will get them); 0 for one f32 row of Q8_0 / Q4_0 that its kernel quantizes (the
+ * workspace pointer must be valid all the same).  No reference counterpart: Candle allocates
+ * inside forward. */
 sxq_status sxq_qmm_workspace_size(const sxq_qmm *qmm, int64_t m, unsigned flags, size_t *bytes);
 
 /* QMatMul::forward exactly as sxq_qmm_forward (same checks, kernels and bits), on device
