@@ -22,9 +22,10 @@
 //    Eight times the parallelism per tile at about twice the work per output: for few tiles.
 // One kernel (64 x 128 tiles, operands one block ahead in registers, 1.1 us per block) for 128
 // rows and more and the GEMV four rows per launch below took: 896 x 4864 at 8 / 50 / 226 rows
-// 12.9 / 69 / 166 us (now 10.8 / 11.4 / 21.0), 9728 x 896 12.5 / 63 / 45 (7.6 / 10.4 / 20.6), 2048 x
+// 12.9 / 69 / 166 us (now 10.8 / 11.4 / 21.3), 9728 x 896 12.5 / 63 / 45 (7.6 / 10.4 / 20.6), 2048 x
 // 1024 Q4_0 at 500 rows 46.7 (14.7), all with the activation quantizer's launch.
 #include "sxq_kernels.h"
+#include "sxq_q80_stage.h"
 #include "sxq_quant_dev.h"
 
 namespace sxq {
@@ -389,8 +390,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80(const ActQ8_0* __restrict__
 
 // ---- in between: one wave per 16 x 16 tile ----------------------------------------------
 
-constexpr int kMdT = 32;  // rows and weight rows per workgroup: 2 x 2 waves
-constexpr int kMdKC = 8;  // blocks per LDS stage
+static_assert(kMdActB == sizeof(ActQ8_0), "an activation block");
 
 // The same chains in registers over 16 x 16 tiles (v_mfma_i32_16x16x32_i8, lanes as in the
 // split kernel): a quarter of the per-block time, four times the tiles.  Stages of eight
@@ -418,34 +418,32 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
     // staging roles: pieces p and p + 8 (blocks p / 2 and p / 2 + 4) of row pr; block jb of row
     // jr (scales, Q4_0 blocks)
     const int pr = tid >> 3, p = tid & 7, jr = tid >> 3, jb = tid & 7;
-    // A thread's offsets into the tile's rows stay; a stage only moves the scalar offset.  What
-    // lies past the tile's rows loads as zero, what lies past a row is the next one's: neither
-    // is added or stored.
     const int rm = min(kMdT, M - m0), rn = min(kMdT, N - n0);
-    constexpr uint32_t AB = sizeof(ActQ8_0), WB = Q4 ? 16 : 32;
     auto rsrc = [](const void* p, uint32_t bytes) {
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
     };
-    const __amdgpu_buffer_rsrc_t ars = rsrc(act + (int64_t)m0 * nb, (uint32_t)(rm * nb) * AB);
+    constexpr uint32_t WB = Q4 ? 16 : 32;
+    const __amdgpu_buffer_rsrc_t ars = rsrc(act + (int64_t)m0 * nb, (uint32_t)(rm * nb) * kMdActB);
     const __amdgpu_buffer_rsrc_t wrs = rsrc(wqs + (int64_t)n0 * nb * WB, (uint32_t)(rn * nb) * WB);
     const __amdgpu_buffer_rsrc_t drs = rsrc(wd + (int64_t)n0 * nb, (uint32_t)(rn * nb) * 2u);
-    const uint32_t oa = (uint32_t)(pr * nb + (p >> 1)) * AB + 16u * (p & 1), oda = (uint32_t)(jr * nb + jb) * AB + 32u;
-    const uint32_t ow = Q4 ? (uint32_t)(jr * nb + jb) * 16u : (uint32_t)(pr * nb + (p >> 1)) * 32u + 16u * (p & 1);
-    const uint32_t odw = (uint32_t)(jr * nb + jb) * 2u;
     struct Regs {
         v4i a[2], b[2];
         float da;
         uint16_t dw;
     };
+    // A thread's offsets stay; a stage only moves the scalar offset, and the stages at the row's end
+    // (the last one, and the two loaded ahead of it) stop at the row's last eight blocks.
+    const MidLoads o = mid_loads<Q4>(tid, rm, rn, nb);
     auto load = [&](Regs& k, int c0) {
+        const uint32_t b = (uint32_t)mid_first(c0, nb);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            k.a[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ars, oa + 4 * i * AB, c0 * AB, 0));
-            if (!Q4) k.b[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, ow + 128u * i, c0 * WB, 0));
+            k.a[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ars, o.a[i], b * kMdActB, 0));
+            if (!Q4 || i == 0)
+                k.b[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, o.w[i], b * WB, 0));
         }
-        k.da = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ars, oda, c0 * AB, 0));
-        k.dw = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(drs, odw, c0 * 2, 0);
-        if (Q4) k.b[0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, ow, c0 * WB, 0));
+        k.da = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ars, o.da, b * kMdActB, 0));
+        k.dw = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(drs, o.dw, b * 2u, 0);
     };
     auto slot = [](int row, int piece) { return row * 256 + ((piece ^ (row & 15)) << 4); };
     auto store = [&](const Regs& k, int st) {
@@ -489,7 +487,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
     };
     // Four blocks' operands are read and multiplied together, and the next four read while
     // they are folded: a wave often has its SIMD to itself, and block by block it waited for
-    // LDS and the matrix cores at each (896 x 4864 at 226 rows 24.9 us, now 21.0).
+    // LDS and the matrix cores at each (896 x 4864 at 226 rows 24.9 us, now 21.3).
     auto compute = [&](int st, int c) {
         const int kc = nb - c * kMdKC;
         if (kc >= kMdKC) {
@@ -511,9 +509,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
 #pragma unroll
             for (int j = 0; j < 4; ++j) fold(n[j], s[j]);
         } else {
+            const int c0 = c * kMdKC, slot0 = c0 - mid_first(c0, nb);
             for (int j = 0; j < kc; ++j) {
                 Block k;
-                read(k, st, j);
+                read(k, st, slot0 + j);
                 fold(k, dots(k));
             }
         }
@@ -524,9 +523,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
     load(r0, 0);
     load(r1, kMdKC);
     store(r0, 0);
+    __builtin_amdgcn_sched_barrier(0);  // r1's loads stay ahead of r0's, or the loop waits for both at once
     load(r0, 2 * kMdKC);
     lds_barrier();
-    for (int c = 0; c < nc; c += 2) {
+    for (int c = 0;; c += 2) {
         compute(0, c);
         if (c + 1 >= nc) break;  // uniform
         store(r1, 1);            // stage buffers: read last a stage ago, behind a barrier
