@@ -126,13 +126,12 @@ sxq_status sxq_qmm_forward(const sxq_qmm *qmm, const float *x, const int64_t *x_
 
 /* Device workspace bytes sxq_qmm_forward_ws needs for m rows of x (with `flags` as the
  * forward will get them); 0 for one f32 row of Q8_0 / Q4_0 that its kernel quantizes (the
- * workspace pointer must be valid all the same).  No reference counterpart: Candle allocates
- * inside forward. */
+ * workspace may then be NULL).  No reference counterpart: Candle allocates inside forward. */
 sxq_status sxq_qmm_workspace_size(const sxq_qmm *qmm, int64_t m, unsigned flags, size_t *bytes);
 
 /* QMatMul::forward exactly as sxq_qmm_forward (same checks, kernels and bits), on device
  * pointers, with a caller-provided device workspace (`workspace_bytes` >=
- * sxq_qmm_workspace_size, 256-byte aligned) instead of the library's shared one: for
+ * sxq_qmm_workspace_size, 256-byte aligned; not looked at where that is 0) instead of the library's shared one: for
  * code under graph capture (the graph owns the workspace, so replays never alias other
  * calls) and callers that manage their own memory.  Calls that share one workspace
  * must not overlap.  flags: SXQ_BIT_EXACT, SXQ_BF16_INPUT. */

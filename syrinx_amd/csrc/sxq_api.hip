@@ -443,10 +443,10 @@ sxq_status sxq_qmm_forward_ws(const sxq_qmm* q, const float* x, const int64_t* s
     if (st != SXQ_OK) return st;
     if (p.m == 0) return SXQ_OK;
     if (!x || !y) return fail(SXQ_ERR_INVALID, "qmm_forward_ws: null x or y");
-    if (workspace_bytes < p.ws || !workspace)
+    if (p.ws > 0 && (workspace_bytes < p.ws || !workspace))
         return fail(SXQ_ERR_INVALID, "qmm_forward_ws: the workspace holds %zu bytes, this call needs %zu",
                     workspace ? workspace_bytes : (size_t)0, p.ws);
-    if ((uintptr_t)workspace & 255) return fail(SXQ_ERR_INVALID, "qmm_forward_ws: workspace not 256-byte aligned");
+    if (p.ws > 0 && ((uintptr_t)workspace & 255)) return fail(SXQ_ERR_INVALID, "qmm_forward_ws: workspace not 256-byte aligned");
     DeviceGuard g(q->device);
     HIP_TRY(g.err, "hipSetDevice");
     HIP_TRY(run_forward(q, p, x, y, bias, (uint8_t*)workspace, (hipStream_t)stream), "qmm_forward_ws");

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from syrinx_amd import GgmlDType, QMatMul, QTensor
-from syrinx_amd._lib import check, lib
+from syrinx_amd._lib import BF16_INPUT, ERR_INVALID, check, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -167,6 +167,35 @@ def test_forward_workspaces(cuda, dt, k, m):
         eager = qmm.forward(xs[5])
         torch.cuda.synchronize()
         assert torch.equal(y, w) and torch.equal(eager, want[5])
+
+
+@pytest.mark.parametrize("dt,k", [(G.Q4K, 512), (G.Q8_0, 896), (G.Q4_0, 320)])
+@pytest.mark.parametrize("m", [1, 2])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_queried_workspace_is_enough(cuda, dt, k, m, bf16):
+    """The C sequence of a caller with its own memory: query the size, allocate that many bytes
+    (a null pointer for none), run; one byte less is refused where any is needed."""
+    gen = torch.Generator(device=cuda).manual_seed(k + m)
+    qmm = QMatMul.from_qtensor(QTensor.quantize(torch.randn(300, k, generator=gen, device=cuda) * 0.02, dt))
+    x = torch.randn(m, k, generator=gen, device=cuda)
+    x = x.bfloat16() if bf16 else x
+    flags = BF16_INPUT if bf16 else 0
+    need = ctypes.c_size_t()
+    check(lib().sxq_qmm_workspace_size(qmm._h, m, flags, ctypes.byref(need)))
+    assert need.value > 0 or (m == 1 and dt != G.Q4K and not bf16)
+    ws = torch.empty(need.value, dtype=torch.uint8, device=cuda)
+    y = torch.zeros(m, 300, device=cuda)
+
+    def run(nbytes):
+        return lib().sxq_qmm_forward_ws(qmm._h, ctypes.c_void_p(x.data_ptr()), (ctypes.c_int64 * 2)(m, k), 2, None,
+                                        ctypes.c_void_p(y.data_ptr()), None, flags,
+                                        ctypes.c_void_p(ws.data_ptr() if nbytes else None), nbytes,
+                                        torch.cuda.current_stream().cuda_stream)
+
+    check(run(need.value))
+    assert torch.equal(y, qmm.forward(x))
+    if need.value:
+        assert run(need.value - 1) == ERR_INVALID and run(0) == ERR_INVALID
 
 
 @pytest.mark.parametrize("dim,inter,T", [(256, 512, 64), (1280, 4352, 65), (4352, 256, 257)])
