@@ -754,21 +754,21 @@ SXQ_DEV half8_t mma_act8(uint2 v) {
 }
 
 __global__ __launch_bounds__(512) void k_gemv_mma_q4k(const uint4* __restrict__ hdr, const uint4* __restrict__ qs,
-                                                      int n, int nb, const uint8_t* __restrict__ act, int m, int slabs,
+                                                      int n, int nb, const uint8_t* __restrict__ act, int m, int gx,
                                                       float* y, int64_t ldy, const float* __restrict__ bias,
                                                       const float* res, int64_t ldr) {
     extern __shared__ uint4 lds[];
     uint32_t* l32 = (uint32_t*)lds;  // [2][kMmaBuf]: weights [16][kMmaWRow], headers [16][4] uint4, act [16][kMmaARow]
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int g = lane >> 4, nl = lane & 15;
-    // workgroup id -> (16-row slab of x, weight tile): the slabs of one weight tile run on the
-    // same XCD (id mod 8), close together, so its L2 serves their re-reads of the weights
-    const int slot = blockIdx.x >> 3, slab = slot % slabs;
-    const int row0 = ((slot / slabs) * 8 + (blockIdx.x & 7)) * kMmaRows;
-    if (row0 >= n) return;  // uniform: padding of the weight tiles to a multiple of 8
+    // Grid (gx, slabs of 16 rows of x, weight tiles / gx): with several slabs gx is 8, so those of
+    // one weight tile run on the same XCD (workgroup id mod 8), close together, and its L2 serves
+    // their re-reads of the weights; one slab has the tiles in x.  (One dimension and a division
+    // by the slab count delayed every first load: 6144 x 2560 at 5..16 rows 11.1 us, now 10.7,
+    // 155776 x 2560 125.7, now 123.7.)
+    const int slab = blockIdx.y;
+    const int row0 = ((int)blockIdx.z * gx + (int)blockIdx.x) * kMmaRows;
     act += (size_t)slab * 16 * nb * sizeof(ActQ8K);
-    y += (int64_t)slab * 16 * ldy;
-    if (res) res += (int64_t)slab * 16 * ldr;
     m = min(16, m - 16 * slab);
     const int nc = (nb + kMmaChunk - 1) / kMmaChunk;
 
@@ -837,6 +837,8 @@ __global__ __launch_bounds__(512) void k_gemv_mma_q4k(const uint4* __restrict__ 
     stage_store(0);
     stage_load(1);
     __syncthreads();
+    if (row0 >= n) return;  // uniform: padding of the weight tiles to a multiple of gx (here, so
+                            // that the first loads do not wait for n)
     for (int c = 0; c < nc; ++c) {
         const uint32_t* bw = l32 + (c & 1) * kMmaBuf;
         const uint4* bh = (const uint4*)(bw + 16 * kMmaWRow);
@@ -895,8 +897,9 @@ __global__ __launch_bounds__(512) void k_gemv_mma_q4k(const uint4* __restrict__ 
         for (int cl = 0; cl < 8; ++cl) tot += xb[cl * 256 + tid];
         float v = xb[8 * 256 + tid] + tot;
         if (bias) v = v + bias[row];
-        if (res) v = res[(int64_t)mr * ldr + row] + v;
-        y[(int64_t)mr * ldy + row] = v;
+        const int64_t xr = 16 * slab + mr;
+        if (res) v = res[xr * ldr + row] + v;
+        y[xr * ldy + row] = v;
     }
 }
 
@@ -1176,10 +1179,10 @@ static hipError_t gemv_mma_launch(const QWeight& w, const void* act, int m, floa
         hipFuncSetAttribute((const void*)k_gemv_mma_q4k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMmaLds);
     if (attr != hipSuccess) return attr;
     const int n = (int)w.n, nb = (int)w.nb;
-    const int tiles = (n + kMmaRows - 1) / kMmaRows, slabs = (m + 15) / 16;
-    hipLaunchKernelGGL(k_gemv_mma_q4k, dim3((unsigned)((tiles + 7) / 8 * 8 * slabs)), dim3(512), kMmaLds, s,
-                       (const uint4*)w.hdr, (const uint4*)w.qs, n, nb, (const uint8_t*)act, m, slabs, y, ldy, bias, res,
-                       ldr);
+    const int tiles = (n + kMmaRows - 1) / kMmaRows, slabs = (m + 15) / 16, gx = slabs == 1 ? tiles : 8;
+    hipLaunchKernelGGL(k_gemv_mma_q4k, dim3((unsigned)gx, (unsigned)slabs, (unsigned)((tiles + gx - 1) / gx)), dim3(512),
+                       kMmaLds, s, (const uint4*)w.hdr, (const uint4*)w.qs, n, nb, (const uint8_t*)act, m, gx, y, ldy,
+                       bias, res, ldr);
     return hipGetLastError();
 }
 
@@ -1252,7 +1255,8 @@ hipError_t launch_gemv_rec(const QWeight& w, const void* act, const MmaRec* rec,
 hipError_t launch_gemv(const QWeight& w, const void* act, int m, float* y, int64_t ldy, const float* bias,
                        const float* res, int64_t ldr, hipStream_t s) {
     if (m <= 0 || w.n <= 0) return hipSuccess;
-    if (m > 16 && (w.dtype != kQ4K || gemv_v1() || !gemv_mma_on())) {  // 16 rows at a time
+    // 16 rows at a time, also where the slabs' launch has too few grid rows for the weight tiles
+    if (m > 16 && (gemv_v1() || !gemv_mma_on() || w.n > (int64_t)65535 * 8 * kMmaRows)) {
         const size_t row_bytes = (size_t)w.nb * (block_size(w.dtype) / block_size(vec_dot_type(w.dtype))) *
                                  act_block_bytes(vec_dot_type(w.dtype));
         for (int r0 = 0; r0 < m; r0 += 16) {
@@ -1270,7 +1274,7 @@ hipError_t launch_gemv(const QWeight& w, const void* act, int m, float* y, int64
         if (fits && m == 2) return gemv2_dispatch<2>(w, act, m, y, ldy, bias, res, ldr, s);
         if (fits && m <= 4) return gemv2_dispatch<4>(w, act, m, y, ldy, bias, res, ldr, s);
         // five rows and more of Q4_K: the matrix cores, every 16-row slab in one launch
-        // (6144 x 2560 at 37 rows: 21.9 us, against 3 x 9.2 one launch per slab)
+        // (6144 x 2560 at 37 rows: 20.1 us, 26.2 with one launch per slab)
         if (w.dtype == kQ4K && m > 4 && gemv_mma_on()) return gemv_mma_launch(w, act, m, y, ldy, bias, res, ldr, s);
         if (w.dtype != kQ4K && m >= kGemmQ80MinRows) return launch_gemm_q80(w, act, m, y, ldy, bias, res, ldr, s);
         // 5..16 rows: the task-split kernel four activation rows at a time (each launch
