@@ -1275,7 +1275,25 @@ hipError_t launch_gemv(const QWeight& w, const void* act, int m, float* y, int64
         if (fits && m <= 4) return gemv2_dispatch<4>(w, act, m, y, ldy, bias, res, ldr, s);
         // five rows and more of Q4_K: the matrix cores, every 16-row slab in one launch
         // (6144 x 2560 at 37 rows: 20.1 us, 26.2 with one launch per slab)
-        if (w.dtype == kQ4K && m > 4 && gemv_mma_on()) return gemv_mma_launch(w, act, m, y, ldy, bias, res, ldr, s);
+        if (w.dtype == kQ4K && m > 4 && gemv_mma_on()) {
+            // One to three rows past the last whole slab: a slab of their own costs as much as a
+            // full one.  On wide weights, whose slabs run one generation of workgroups after
+            // another, the GEMV of those rows is the shorter end: from 512 weight tiles for one
+            // row (8192 x 2560 at 17 rows 17.4 -> 15.0 us, 155776 x 2560 242 -> 161; at 384 tiles,
+            // 6144 x 2560, 14.9 / 14.5 at 17 rows and 23.7 / 24.1 at 49), from 768 for two (12288 x
+            // 2560 at 18 rows 23.4 -> 21.5; 8192 x 1024 11.0 / 12.0), from 1024 for three (19456 x
+            // 2560 at 19 rows 35.6 -> 34.0; 12288 x 2560 23.1 / 23.1).  Four take as long as a slab
+            // (19456 x 2560 at 20 rows 36.0 / 36.6).
+            const int odd = m % 16, tiles = (int)((w.n + kMmaRows - 1) / kMmaRows);
+            const bool alone = odd >= 1 && odd <= 3 && tiles >= 256 * (odd + 1);
+            if (m < 16 || !alone || !gemv2_fits((int)w.n, nb, odd, w.dtype, 256))
+                return gemv_mma_launch(w, act, m, y, ldy, bias, res, ldr, s);
+            const int64_t m0 = m - odd;
+            const hipError_t e = gemv_mma_launch(w, act, (int)m0, y, ldy, bias, res, ldr, s);
+            if (e != hipSuccess) return e;
+            return launch_gemv(w, (const uint8_t*)act + (size_t)m0 * nb * sizeof(ActQ8K), odd, y + m0 * ldy, ldy, bias,
+                               res ? res + m0 * ldr : nullptr, ldr, s);
+        }
         if (w.dtype != kQ4K && m >= kGemmQ80MinRows) return launch_gemm_q80(w, act, m, y, ldy, bias, res, ldr, s);
         // 5..16 rows: the task-split kernel four activation rows at a time (each launch
         // streams the weights again; per row this is still well ahead of the

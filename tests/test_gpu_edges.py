@@ -75,7 +75,10 @@ def test_q80_matrix_core_bit_exact(cuda, ora, dt, n, k, m):
     assert (got == want).all(), f"{int((got != want).sum())} of {got.size} outputs differ"
 
 
-@pytest.mark.parametrize("n,k,m", [(7, 256, 17), (40, 1536, 33), (1003, 2560, 63), (6144, 512, 48), (130, 1024, 21)])
+@pytest.mark.parametrize("n,k,m", [(7, 256, 17), (40, 1536, 33), (1003, 2560, 63), (6144, 512, 48), (130, 1024, 21),
+                                   # one to three rows past the last slab, around the widths from which they run alone
+                                   (8170, 512, 17), (8177, 512, 33), (12270, 256, 18), (12280, 256, 50), (16360, 256, 19),
+                                   (16370, 256, 35)])
 def test_q4k_slabs_bit_exact(cuda, ora, n, k, m):
     """17..63 rows of Q4_K (and any count with exact=True): every 16-row slab of one launch, a
     partial last slab, weight tiles that are no multiple of eight."""
