@@ -40,7 +40,7 @@ inline size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 // One QMatMul::forward, checked: m rows of x, which kernel family, workspace bytes.
 struct FwdPlan {
     int64_t m = 0;
-    bool gemm = false;  // the MFMA prefill GEMM (else quantized activations + GEMV)
+    bool gemm = false;  // Q4_K's f16 prefill GEMM (else quantized activations and launch_gemv)
     int vdt = 0;
     int64_t nbv = 0;    // activation blocks per row
     size_t ws = 0;      // device workspace: activation blocks, or the GEMM's staging

@@ -326,22 +326,20 @@ sxq_status plan_forward(const sxq_qmm* q, const int64_t* shape, int ndim, const 
     p->m = m;
     p->vdt = vec_dot_type(q->w.dtype);
     p->nbv = q->w.k / block_size(p->vdt);
-    // Many rows: a GEMM, one pass over the weights.  Q8_0 / Q4_0 run the int8 matrix-core
-    // GEMM, bit-identical to Candle's vec-dot.  Q4_K runs the f16 MFMA GEMM (operands
-    // rounded to f16, error below 2^-10 * sum |w x| per output) unless SXQ_BIT_EXACT asks
-    // for Candle's integer vec-dot (the GEMV, 16 rows at a time).
-    const bool q80 = q->w.dtype == kQ8_0 || q->w.dtype == kQ4_0;
-    p->gemm = q80 ? m >= kGemmQ80MinRows : (m >= kGemmMinRows && !(flags & SXQ_BIT_EXACT));
+    // Many rows of Q4_K: the f16 MFMA GEMM (operands rounded to f16, error below
+    // 2^-10 * sum |w x| per output) unless SXQ_BIT_EXACT asks for Candle's integer vec-dot.
+    // Everything else is Candle's bits (launch_gemv, which chooses the kernel).
+    p->gemm = q->w.dtype == kQ4K && m >= kGemmMinRows && !(flags & SXQ_BIT_EXACT);
     // one row that its GEMV quantizes needs none
     const bool row = m == 1 && fused_quant(q->w);
     p->ws = m == 0 || row ? 0
-                          : up256(p->gemm && !q80 ? gemm_q4k_workspace(q->w.n, (int)m, q->w.k)
+                          : up256(p->gemm ? gemm_q4k_workspace(q->w.n, (int)m, q->w.k)
                                                   : (size_t)m * (size_t)p->nbv * act_block_bytes(p->vdt));
     // bf16 input: the quantizer reads it (an exact widening in registers: no launch and no f32
     // copy of x).  The f16 GEMM and the one-row GEMV that quantizes in its prologue take f32
     // rows: widened to f32 at the workspace's end, then the f32 forward.
     p->bf16 = (flags & SXQ_BF16_INPUT) && m > 0;
-    const bool f32_rows = (p->gemm && !q80) || row;
+    const bool f32_rows = p->gemm || row;
     p->xconv = p->bf16 && f32_rows ? up256((size_t)m * (size_t)q->w.k * 4) : 0;
     p->ws += p->xconv;
     return SXQ_OK;
@@ -356,7 +354,7 @@ hipError_t run_forward(const sxq_qmm* q, const FwdPlan& p, const float* x, float
         if (e != hipSuccess) return e;
         x = xf;
     }
-    if (p.gemm && q->w.dtype == kQ4K) {
+    if (p.gemm) {
         hipError_t e = launch_gemm_q4k_prep(x, k, (int)m, n, (int)k, ws, s);
         if (e == hipSuccess) e = launch_gemm_q4k(q->w, ws, (int)m, y, n, bias, nullptr, 0, s);
         return e;
@@ -365,9 +363,7 @@ hipError_t run_forward(const sxq_qmm* q, const FwdPlan& p, const float* x, float
     if (m == 1 && fused_quant(q->w)) return launch_gemv_quant(q->w, x, y, bias, nullptr, s);
     hipError_t e = p.bf16 ? launch_quantize_act_bf16(p.vdt, (const uint16_t*)(const void*)x, k, (int)m, (int)k, ws, s)
                           : launch_quantize_act(p.vdt, false, x, k, (int)m, (int)k, ws, s);
-    if (e != hipSuccess) return e;
-    return p.gemm ? launch_gemm_q80(q->w, ws, (int)m, y, n, bias, nullptr, 0, s)
-                  : launch_gemv(q->w, ws, (int)m, y, n, bias, nullptr, 0, s);
+    return e == hipSuccess ? launch_gemv(q->w, ws, (int)m, y, n, bias, nullptr, 0, s) : e;
 }
 
 }  // namespace abi

@@ -1256,7 +1256,8 @@ hipError_t launch_gemv(const QWeight& w, const void* act, int m, float* y, int64
                        const float* res, int64_t ldr, hipStream_t s) {
     if (m <= 0 || w.n <= 0) return hipSuccess;
     // 16 rows at a time, also where the slabs' launch has too few grid rows for the weight tiles
-    if (m > 16 && (gemv_v1() || !gemv_mma_on() || w.n > (int64_t)65535 * 8 * kMmaRows)) {
+    const bool slabs = w.dtype != kQ4K || (gemv_mma_on() && w.n <= (int64_t)65535 * 8 * kMmaRows);
+    if (m > 16 && (gemv_v1() || !slabs)) {
         const size_t row_bytes = (size_t)w.nb * (block_size(w.dtype) / block_size(vec_dot_type(w.dtype))) *
                                  act_block_bytes(vec_dot_type(w.dtype));
         for (int r0 = 0; r0 < m; r0 += 16) {
@@ -1294,10 +1295,16 @@ hipError_t launch_gemv(const QWeight& w, const void* act, int m, float* y, int64
             return launch_gemv(w, (const uint8_t*)act + (size_t)m0 * nb * sizeof(ActQ8K), odd, y + m0 * ldy, ldy, bias,
                                res ? res + m0 * ldr : nullptr, ldr, s);
         }
-        if (w.dtype != kQ4K && m >= kGemmQ80MinRows) return launch_gemm_q80(w, act, m, y, ldy, bias, res, ldr, s);
-        // 5..16 rows: the task-split kernel four activation rows at a time (each launch
-        // streams the weights again; per row this is still well ahead of the
-        // one-group-per-row kernel, whose few waves leave most of the GPU idle).
+        // five rows and more of Q8_0 / Q4_0: the int8 matrix cores, but for up to eight rows of a
+        // long K over few outputs, where a workgroup's chunks are a longer chain than two GEMV
+        // launches (us, split kernel / GEMVs at 5 and 8 rows: 128 x 8192 14.5 / 12.4 and 14.5 /
+        // 13.7; 512 x 8192 14.6 / 13.4 and 14.5 / 14.4; 768 x 8192 14.5 / 14.5 and 14.6 / 15.4;
+        // 128 x 7168 13.2 / 11.8 and 13.3 / 13.1; 128 x 6144 11.9 / 11.3 and 12.0 / 12.3)
+        const bool few = m <= 8 && w.n <= 512 && nb >= 224 && gemv2_fits((int)w.n, nb, 4, w.dtype, 256);
+        if (w.dtype != kQ4K && m >= 5 && !few) return launch_gemm_q80(w, act, m, y, ldy, bias, res, ldr, s);
+        // those, and Q4_K without its matrix-core kernel: the task-split kernel four activation
+        // rows at a time (each launch streams the weights again; per row this is still well
+        // ahead of the one-group-per-row kernel, whose few waves leave most of the GPU idle).
         if (m <= 16 && gemv2_fits((int)w.n, nb, 4, w.dtype, 256)) {
             const size_t row_bytes = (size_t)nb * act_block_bytes(vec_dot_type(w.dtype));
             for (int r0 = 0; r0 < m; r0 += 4) {

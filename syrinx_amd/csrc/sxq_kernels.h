@@ -95,7 +95,6 @@ hipError_t launch_swiglu_pair(const QWeight& gate_up, const QWeight& down, const
 // f16 in the GEMM's K order and, when K is split across workgroups, the partial tiles
 // and their counters; launch_gemm_q4k_prep fills it from x, then launch_gemm_q4k runs.
 constexpr int kGemmMinRows = 64;  // QMatMul::forward uses the Q4_K GEMM from this many rows on
-constexpr int kGemmQ80MinRows = 5;  // ... and the Q8_0 / Q4_0 matrix-core kernels (below: the GEMV)
 size_t gemm_q4k_workspace(int64_t n, int m, int64_t k);
 hipError_t launch_gemm_q4k_prep(const float* x, int64_t ldx, int m, int64_t n, int k, void* ws, hipStream_t s);
 // The same workspace from rows that are still to be computed, for k <= kPrepMaxK: the RMSNorm

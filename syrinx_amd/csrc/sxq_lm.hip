@@ -417,8 +417,7 @@ sxq_status check_config(const sxq_lm_config* c) {
 
 // One projection of T prompt rows: x_f32 [T][k] (f32 rows) and act (the same rows as
 // device activation blocks) -> y [T][n] (+ bias, then res + that).  Q4_K: the f16 MFMA GEMM
-// from kGemmMinRows rows unless `exact`; Q8_0 / Q4_0: the int8 matrix cores from
-// kGemmQ80MinRows rows; otherwise the GEMV (Candle's bits).
+// from kGemmMinRows rows unless `exact`; otherwise Candle's bits (launch_gemv).
 hipError_t pf_proj(const sxq_lm* lm, const QWeight& w, const float* x, const uint8_t* act, int T, float* y,
                    const float* bias, const float* res, bool exact, void* gemm_ws, hipStream_t s) {
     const int64_t n = w.n;
@@ -426,7 +425,6 @@ hipError_t pf_proj(const sxq_lm* lm, const QWeight& w, const float* x, const uin
         hipError_t e = launch_gemm_q4k_prep(x, w.k, T, n, (int)w.k, gemm_ws, s);
         return e == hipSuccess ? launch_gemm_q4k(w, gemm_ws, T, y, n, bias, res, n, s) : e;
     }
-    if (w.dtype != kQ4K && T >= kGemmQ80MinRows) return launch_gemm_q80(w, act, T, y, n, bias, res, n, s);
     return launch_gemv(w, act, T, y, n, bias, res, n, s);
 }
 

@@ -50,11 +50,13 @@ def test_quantize_rows_remainders_and_unaligned(cuda, ora, dt, k, n, shift):
 
 
 # (n, k, m): weight tiles of 16 / 64 / 128 rows and row tiles of 16 / 32 / 64 with remainders,
-# block counts below, at and past a chunk (4, 8, 16, 32 blocks), each kernel of the dispatch
+# block counts below, at and past a chunk (4, 8, 16, 32 blocks)
 Q80_SHAPES = [(1, 32, 5), (17, 320, 16), (16, 1024, 17), (130, 1056, 33), (896, 4864, 8), (77, 992, 64), (200, 160, 65),
               (1152, 896, 226), (2048, 1024, 500), (4100, 96, 130), (896, 4864, 226), (9728, 896, 50), (64, 2080, 300),
               # 32 x 32 tiles whose last row tile and weight tile hold one row: 1, 10 and 28 blocks
-              (2049, 32, 97), (2049, 320, 97), (1153, 896, 225)]
+              (2049, 32, 97), (2049, 320, 97), (1153, 896, 225),
+              # a long K over few outputs (the GEMV up to 512 outputs and eight rows)
+              (512, 8192, 6), (40, 7168, 8), (513, 7168, 5), (40, 7168, 9)]
 
 
 @pytest.mark.parametrize("dt", [G.Q8_0, G.Q4_0])
