@@ -13,7 +13,7 @@
 // GEMM (which rounds both operands).  The float fold is 4 VALU instructions per output per
 // block against 1/16 of an MFMA, so with enough tiles the work is bound by VALU issue.
 //
-// The adds of one output are a serial chain over its blocks, and two kernels split the rest:
+// The adds of one output are a serial chain over its blocks, and three kernels split the rest:
 //  * k_gemm_q80: one wave per 32 x 32 tile, the chain in its registers; ~0.27 us per block
 //    where a SIMD holds one wave, so this is for shapes with many tiles.
 //  * k_gemm_q80_mid: one wave per 16 x 16 tile, likewise: four times the waves.
@@ -523,7 +523,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q80_mid(const ActQ8_0* __restri
     load(r0, 0);
     load(r1, kMdKC);
     store(r0, 0);
-    __builtin_amdgcn_sched_barrier(0);  // r1's loads stay ahead of r0's, or the loop waits for both at once
+    // r1's loads stay ahead of r0's: interleaved, a wait for one stage's takes the other's too (the
+    // 226-row CosyVoice2 prompt 2043 us, now 2024)
+    __builtin_amdgcn_sched_barrier(0);
     load(r0, 2 * kMdKC);
     lds_barrier();
     for (int c = 0;; c += 2) {
@@ -567,24 +569,25 @@ static hipError_t gemm_q80_dispatch(const QWeight& w, const ActQ8_0* act, int m,
                            tm, tn, y, ldy, bias, res, ldr);                                                  \
         return hipGetLastError();                                                                            \
     } while (0)
-    // The kernel by the number of 16 x 16 tiles, T, and of 64 x 64 tiles (us with the
-    // activation quantizer's launch, in a graph; split by blocks / mid / 64 x 64, before each of
-    // them became 3 to 15 % faster):
-    //  T <= 256, a workgroup per CU: the split kernel with 32-block chunks (896 x 4864 at 64
-    //  rows, T = 224: 12.9 / 22.6 / 48; 2048 x 1024 Q4_0 at 32 rows, T = 256: 6.4 / 9.1 / 16);
-    //  T <= 768: with 16-block chunks, three workgroups per CU (9728 x 896 at 16 rows, T = 608:
-    //  8.6 / 9.8 / 13.8; 2560 x 9728 at 50 rows, T = 640: 37.1 / 40.2 / 89.5; 2048 x 1024 at 128
-    //  rows, T = 1024: 10.0 / 9.5 / 16.4);
-    //  fewer than 400 64 x 64 tiles: mid (2048 x 1024 at 500 rows, 256 tiles: 25.4 / 14.3 / 18.3;
-    //  9728 x 896 at 128 rows, 304: 28.6 / 16.4 / 18.2; 2560 x 9728 at 500, 320: 215 / 106 / 115);
-    //  from there on 64 x 64 (6564 x 896 at 226 rows, 412 tiles: 36.6 / 20.2 / 19.0; 9728 x 896 at
-    //  500 rows, 1216 tiles: 101 / 45.4 / 35.8).
+    // The kernel by the number of 16 x 16 tiles, T, and of 64 x 64 tiles, T64 (us with the
+    // activation quantizer's launch, in a graph):
+    //  T <= 256, a workgroup per CU: the split kernel with 32-block chunks (split 32 / split 16 /
+    //  mid: 896 x 4864 at 64 rows, T = 224: 12.0 / 12.8 / 18.8, at 65 rows, T = 280: 18.8 / 16.4 /
+    //  18.7; 2048 x 1024 at 32 rows, T = 256: 5.8 / 6.1 / 7.7, at 33 rows, T = 384: 7.8 / 7.0 / 7.8).
+    //  T <= 512, two per CU: with 16-block chunks (split 16 / mid: 2560 x 9728 at 48 rows, T = 480:
+    //  27.2 / 32.4, at 49 rows, T = 640: 34.9 / 32.6; 896 x 4864 at 144 rows, T = 504: 17.6 / 19.7, at
+    //  145 rows, T = 560: 21.5 / 19.6), and up to three per CU for 16 rows, where half of each of
+    //  mid's row tiles is padding (12288 x 896, T = 768: 8.0 / 8.9; 16384 x 2560, T = 1024: 16.2 / 15.7).
+    //  T64 < 400, or one row tile of 32: mid (mid / 64 x 64: 4864 x 896 at 226 rows, T64 = 304: 14.9 /
+    //  16.0, at 300 rows, 380: 16.9 / 16.3; 6564 x 896 at 200 rows, 412: 16.6 / 16.2; 2560 x 9728 at 600
+    //  rows, 400: 99 / 107, at 640 rows: 114 / 107; 1152 x 896 at 1500 rows, 432: 22.8 / 22.1; 151936 x
+    //  896 at 32 rows 43.0 / 49.5, at 33 rows 71.7 / 49.7); from there on 64 x 64.
     // One wave per 32 x 64 tile was never ahead of 32 x 32 (9728 x 896 at 1024 rows: 70.8 against
     // 67.5), nor the split kernel with 32 rows per workgroup ahead of both others.
     const int64_t T = (int64_t)tiles(m, 16) * tiles(N, kSpN);
     if (T <= 256) SXQ_Q80((k_gemm_q80_split<Q4, 4>), 512, 16, kSpN, (SplitShape<Q4, 4>::lds));
-    if (T <= 768) SXQ_Q80((k_gemm_q80_split<Q4, 2>), 512, 16, kSpN, (SplitShape<Q4, 2>::lds));
-    if ((int64_t)tiles(m, kQBM) * tiles(N, kQBM) < 400) SXQ_Q80((k_gemm_q80_mid<Q4>), 256, kMdT, kMdT, 0);
+    if (T <= (m <= 16 ? 768 : 512)) SXQ_Q80((k_gemm_q80_split<Q4, 2>), 512, 16, kSpN, (SplitShape<Q4, 2>::lds));
+    if (m <= kMdT || (int64_t)tiles(m, kQBM) * tiles(N, kQBM) < 400) SXQ_Q80((k_gemm_q80_mid<Q4>), 256, kMdT, kMdT, 0);
     SXQ_Q80((k_gemm_q80<Q4>), 256, kQBM, kQBM, 0);
 #undef SXQ_Q80
 }

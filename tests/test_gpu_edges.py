@@ -55,8 +55,11 @@ Q80_SHAPES = [(1, 32, 5), (17, 320, 16), (16, 1024, 17), (130, 1056, 33), (896, 
               (1152, 896, 226), (2048, 1024, 500), (4100, 96, 130), (896, 4864, 226), (9728, 896, 50), (64, 2080, 300),
               # 32 x 32 tiles whose last row tile and weight tile hold one row: 1, 10 and 28 blocks
               (2049, 32, 97), (2049, 320, 97), (1153, 896, 225),
-              # a long K over few outputs (the GEMV up to 512 outputs and eight rows)
-              (512, 8192, 6), (40, 7168, 8), (513, 7168, 5), (40, 7168, 9)]
+              # 400 tiles of 64 x 64 and more: remainders of rows, weight rows and blocks (3, 29, 5)
+              (6565, 96, 257), (6564, 928, 226), (25700, 160, 33),
+              # the lines of the dispatch: one 32-row tile of a wide weight, 16 rows of 513 tiles, 17 rows of
+              # 514, a long K over few outputs (the GEMV up to 512 outputs and eight rows)
+              (25700, 160, 32), (8200, 96, 9), (4112, 96, 17), (512, 8192, 6), (40, 7168, 8), (513, 7168, 5), (40, 7168, 9)]
 
 
 @pytest.mark.parametrize("dt", [G.Q8_0, G.Q4_0])
