@@ -88,7 +88,7 @@ __global__ __launch_bounds__(1024) void k_rmsnorm_quant(const float* __restrict_
 // rows alone spread over the chip.  Float4 i of the row sits in thread i mod 256, so wave w holds
 // chunks w, w + 4, ... whole; its sums of them are the wave sums of rmsnorm_sumsq_1024.  2868
 // rows of 896 in 10.7 us, against 28.8 with a workgroup of 1024 threads per chunk, each reducing
-// the whole row (226 rows: 4.8 both, the launch's latency).
+// the whole row; fewer rows at kRmsRows.
 template <int VDT>
 __global__ __launch_bounds__(256) void k_rmsnorm_quant_rows(const float* __restrict__ h, int dim,
                                                             const float* __restrict__ w, float inv_n, float eps,
@@ -578,8 +578,10 @@ __global__ void k_fill_int(int* __restrict__ y, int n, int v) {
 }
 
 // ------------------------------------------------------------------------ launchers
-// From this many rows on one workgroup per row is ahead of one per chunk.
-constexpr int kRmsRows = 64;
+// From this many rows on one workgroup per row is ahead of one per chunk (us more per norm within
+// a prompt at 64 / 96 / 128 / 226 rows: dim 896 +0.3 / +0.2 / +0.1 / -1.1, dim 2560 +0.9 / +0.2 /
+// -0.5 / -2.6, in Q8_K +0.6 / -0.1 / -0.7 / -3.1).
+constexpr int kRmsRows = 128;
 hipError_t launch_rmsnorm_quant(int vdt, const float* h, int rows, int dim, const float* w, float eps, uint8_t* act,
                                 float* normed, hipStream_t s, MmaRec* rec) {
     if (rec && (vdt != kQ8K || rows > 16)) return hipErrorInvalidValue;

@@ -908,6 +908,10 @@ def _replay_prefill(ora, lm, cfg, W, tr, counts, lens0, frames, exact):
 PREFILL_KINDS = {
     # name: (config, per-stream (cached length before, prompt tokens), exact)
     "fish_q4k_exact_1stream": (lambda: _fish_small(n_layers=2), [(0, 37)], True),
+    # the RMSNorm quantizer by rows (128 and more), Q8_K, a dim of 2.5 passes of its workgroup
+    "fish_q4k_exact_129_rows": (lambda: D.fish_s2_slow_ar_config(n_layers=1, max_seq=136, vocab=4096, n_codebooks=10,
+                                                                 codebook_size=64, semantic_begin=3000,
+                                                                 semantic_end=4095, intermediate=512), [(3, 129)], True),
     "fish_q4k_gemm_after_cache": (lambda: _fish_small(n_layers=1), [(20, 70)], False),
     "fish_q8_0_ragged3": (lambda: _fish_small(n_layers=2, max_batch=3, dtype=GgmlDType.Q8_0), [(5, 17), (0, 1),
                                                                                                 (31, 40)], True),
