@@ -23,7 +23,7 @@ def cuda():
 
 
 def _rows(n, k, seed):
-    """Normal rows with blocks of zeros, ties, tiny and huge values, infinities and NaN."""
+    """Normal rows with halves of zeros, of one value (ties), tiny and huge values."""
     rng = np.random.default_rng(seed)
     x = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
     for i, v in enumerate((0.0, 0.5, 1e-30, 1e30)):
@@ -47,6 +47,36 @@ def test_quantize_rows_remainders_and_unaligned(cuda, ora, dt, k, n, shift):
     want = ora.quantize(int(dt), x).reshape(-1)
     np.testing.assert_array_equal(got[shift: shift + nbytes], want)
     assert (got[:shift] == 0xA5).all() and (got[shift + nbytes:] == 0xA5).all()
+
+
+def _special_blocks():
+    """[P, 256]: one special pattern each in one of the eight 32-element (sub-)blocks of an otherwise
+    normal row -- infinities and NaN at the first, inner and last lanes of a block, alone, mixed,
+    and over whole blocks and rows; ties of the largest magnitude with either sign first; the
+    largest and subnormal floats; signed zeros."""
+    inf, nan, big = np.float32(np.inf), np.float32(np.nan), np.finfo(np.float32).max
+    pats = [{at: v} for v in (inf, -inf, nan, -nan, big, -big) for at in (0, 5, 31)]
+    pats += [{i: v for i in range(32)} for v in (inf, -inf, nan, big, np.float32(1e-40), np.float32(0.0), np.float32(-0.0))]
+    pats += [{3: inf, 20: -inf}, {20: inf, 3: -inf}, {0: nan, 31: inf}, {31: nan, 0: -inf}, {0: big, 31: -big},
+             {9: 2.0, 2: -2.0}, {9: -2.0, 2: 2.0}, {17: 2.0, 16: -2.0}, {30: 2.0, 1: nan, 4: -2.0}, {7: np.float32(1e-40)},
+             {i: np.float32(-0.0) if i % 3 else np.float32(0.0) for i in range(32)}]
+    x = (np.random.default_rng(11).standard_normal((len(pats) + 3, 256)) * 0.02).astype(np.float32)
+    for p, pat in enumerate(pats):
+        for at, v in pat.items():
+            x[p, 32 * (p % 8) + at] = v
+    x[-3], x[-2] = nan, inf
+    x[-1, ::7] = nan
+    return x
+
+
+@pytest.mark.parametrize("dt", [G.Q8_0, G.Q4_0, G.Q4K])
+def test_quantize_infinities_nan_and_ties(cuda, ora, dt):
+    """The oracle's bytes where a value is not finite or a maximum is tied."""
+    x = _special_blocks()
+    got = QTensor.quantize(torch.from_numpy(x).to(cuda), dt).data().cpu().numpy().reshape(len(x), -1)
+    want = ora.quantize(int(dt), x).reshape(len(x), -1)
+    bad = [int(r) for r in np.flatnonzero((got != want).any(1))]
+    assert not bad, f"rows {bad}: {[(got[r][got[r] != want[r]][:4], want[r][got[r] != want[r]][:4]) for r in bad[:3]]}"
 
 
 # (n, k, m): weight tiles of 16 / 64 / 128 rows and row tiles of 16 / 32 / 64 with remainders,
