@@ -249,9 +249,8 @@ class QMatMul:
         flags = (BIT_EXACT if exact else 0) | (BF16_INPUT if xs.dtype == torch.bfloat16 else 0)
         bptr = _ptr(bias) if bias is not None else None
         need, capturing = ctypes.c_size_t(), torch.cuda.is_current_stream_capturing()
-        rows = xs.numel() // k
-        if strides is None and dims >= 2 and xs.shape[-1] == k and rows <= 65535:
-            check(lib().sxq_qmm_workspace_size(self._h, rows, flags, ctypes.byref(need)))
+        if strides is None and dims >= 2 and xs.shape[-1] == k:
+            check(lib().sxq_qmm_workspace_size(self._h, xs.numel() // k, flags, ctypes.byref(need)))
         if need.value == 0 and not capturing:
             # one row quantized in the kernel's prologue (no workspace), nothing to run, or an
             # argument that the library refuses

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from syrinx_amd import GgmlDType, QMatMul, QTensor
-from syrinx_amd._lib import BF16_INPUT, ERR_INVALID, check, lib
+from syrinx_amd._lib import BF16_INPUT, ERR_INVALID, SxqError, check, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -205,6 +205,13 @@ def test_forward_workspaces(cuda, dt, k, m):
         eager = qmm.forward(xs[5])
         torch.cuda.synchronize()
         assert torch.equal(y, w) and torch.equal(eager, want[5])
+
+
+def test_row_limit_is_the_librarys(cuda):
+    qmm = QMatMul.from_qtensor(QTensor.quantize(torch.ones(1, 32, device=cuda), G.Q8_0))
+    assert qmm.forward(torch.zeros(65535, 32, device=cuda)).shape == (65535, 1)
+    with pytest.raises(SxqError, match="65536 rows exceed the 65535-row limit"):
+        qmm.forward(torch.zeros(2, 32768, 32, device=cuda))
 
 
 @pytest.mark.parametrize("dt,k", [(G.Q4K, 512), (G.Q8_0, 896), (G.Q4_0, 320)])
