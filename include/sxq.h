@@ -119,8 +119,9 @@ sxq_status sxq_qmm_create(int device, int dtype, int64_t n, int64_t k, const voi
  * dimension"), contiguous (x_strides NULL or row-major; else NOT_CONTIGUOUS);
  * y f32 [prod(x_shape[:-1]), n].  Outputs equal Candle's CPU vec-dot bit for bit for
  * every row count of Q8_0 / Q4_0 weights (the decode GEMV up to 4 rows; from 5 rows the
- * int8 matrix cores, which keep Candle's per-block float order), and of Q4_K weights below 64 rows or with SXQ_BIT_EXACT; Q4_K with 64 or more
- * rows runs the f16 MFMA prefill GEMM (error bound at SXQ_BIT_EXACT above). */
+ * int8 matrix cores, which keep Candle's per-block float order), and of Q4_K weights below
+ * 64 rows or with SXQ_BIT_EXACT; Q4_K with 64 or more rows runs the f16 MFMA prefill GEMM
+ * (error bound at SXQ_BIT_EXACT above). */
 sxq_status sxq_qmm_forward(const sxq_qmm *qmm, const float *x, const int64_t *x_shape, int x_ndim,
                            const int64_t *x_strides, float *y, const float *bias, unsigned flags, void *stream);
 

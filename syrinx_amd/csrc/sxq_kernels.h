@@ -106,9 +106,9 @@ hipError_t launch_gemm_q4k_prep_silu(const float* gu, int m, int64_t n, int k, v
 hipError_t launch_gemm_q4k(const QWeight& w, const void* ws, int m, float* y, int64_t ldy, const float* bias,
                            const float* res, int64_t ldr, hipStream_t s);
 
-// Prefill GEMM for Q8_0 / Q4_0 weights (sxq_gemm_q80.hip): the same outputs as the GEMV
-// (Candle's vec-dot, bit for bit) from one pass over the weights on the int8 matrix
-// cores.  act: the Q8_0 activation blocks [m][nb] of launch_quantize_act (device layout).
+// Q8_0 / Q4_0 weights on the int8 matrix cores (sxq_gemm_q80.hip), which launch_gemv takes
+// from five rows on: the GEMV's outputs (Candle's vec-dot, bit for bit).  act: the Q8_0
+// activation blocks [m][nb] of launch_quantize_act (device layout).
 hipError_t launch_gemm_q80(const QWeight& w, const void* act, int m, float* y, int64_t ldy, const float* bias,
                            const float* res, int64_t ldr, hipStream_t s);
 
