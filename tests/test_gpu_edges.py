@@ -79,7 +79,7 @@ def test_quantize_infinities_nan_and_ties(cuda, ora, dt):
     assert not bad, f"rows {bad}: {[(got[r][got[r] != want[r]][:4], want[r][got[r] != want[r]][:4]) for r in bad[:3]]}"
 
 
-# (n, k, m): weight tiles of 16 / 64 / 128 rows and row tiles of 16 / 32 / 64 with remainders,
+# (n, k, m): weight and row tiles of 16 / 32 / 64 rows with remainders,
 # block counts below, at and past a chunk (4, 8, 16, 32 blocks)
 Q80_SHAPES = [(1, 32, 5), (17, 320, 16), (16, 1024, 17), (130, 1056, 33), (896, 4864, 8), (77, 992, 64), (200, 160, 65),
               (1152, 896, 226), (2048, 1024, 500), (4100, 96, 130), (896, 4864, 226), (9728, 896, 50), (64, 2080, 300),
